@@ -1,6 +1,8 @@
-// Error reporting for the C ABI: one message buffer per calling thread.
+// Error reporting for the C ABI (one message buffer per calling thread) and device queries.
 #include <stdarg.h>
 #include <stdio.h>
+
+#include <atomic>
 
 #include "fade_common.h"
 
@@ -30,6 +32,18 @@ int check_launch(const char* what) {
     return FADE_ERUNTIME;
   }
   return FADE_OK;
+}
+
+int num_cus() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cached[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
 }
 
 }  // namespace fade

@@ -15,6 +15,8 @@ void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 int einval(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 // Checks hipGetLastError() after a launch; returns FADE_OK or FADE_ERUNTIME.
 int check_launch(const char* what);
+// Compute units of the current device (256 where the query fails).
+int num_cus();
 
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 

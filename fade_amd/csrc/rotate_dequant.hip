@@ -1,0 +1,385 @@
+// Fused dequantization + rotation back of the rotated backend
+// (fade/rotated_quant.py:134-145,176-187) for fp16 / bf16 output and head_dim 128:
+// out = x_rot @ R with x_rot = dtype(code * scale), read from the packed codes
+// and written once.
+//
+// The two-step path moves x_rot through HBM four times (dequantized rows, an
+// fp32 copy, the fp32 product, the 16-bit copy): 175 us for 33 M elements, of
+// which the fp32 GEMM takes 95.  Here the codes are dequantized in registers
+// into MFMA operands (one rounding to the output type, the reference's) and
+// the product runs on the 16-bit matrix cores with R split so that nothing
+// fp32 holds is lost: fp16 as R_hi + R_lo at a power-of-two scale that puts
+// max|R| in [512, 1024) (~2^-22 of the largest entry), bf16 as three pieces
+// (24 bits); every product accumulates in fp32.
+//
+// MFMA (32x32x16): C^T[out channel][row] = (R^T)[out][in] x_rot^T[in][row].
+// Lane (n, h) of the B operand holds row n, input channels 64 h + 8 ks ..+ 7
+// at step ks: the 64 channels of one lane are contiguous code bytes.  The
+// order within every 8 channels is the one the code conversion produces; R^T
+// is stored in LDS in that order, and its rows so that lane (n, h) receives
+// the 16 consecutive output channels 32 mt + 16 h ..+ 15 of row n.
+//
+// NT row tiles of 32 per wave share every R fragment read from LDS: at NT = 2
+// (fp16) those reads take half the MFMA time instead of all of it.  One
+// workgroup of 16 waves per CU: R's pieces and the output stage fill its LDS,
+// and four waves per SIMD let one's conversions run under another's MFMAs.
+// Measured (4-bit, per call): 16.5 M elements 12 us, 33 M 26.6 us (3.1 TB/s;
+// the two-step path: 168 us), 66 M 55 us (3.0 TB/s).  Up to 33 M elements the
+// split of R in the prologue and the MFMAs bound it, from 66 M the writes (a
+// variant without them: 40 us; without the MFMAs: no faster).
+#include "fade_common.h"
+
+namespace fade {
+namespace {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kD = 128;
+constexpr int kWaves = 16;
+constexpr int kThreads = 64 * kWaves;
+constexpr int kRPitch = 136;  // halves per R^T row in LDS: 16-byte reads of 8 rows hit distinct banks
+constexpr int kStagePitch = 80;  // bytes per staged row of 32 output channels (64 bytes): likewise
+
+// Channel (within its group of 8) that slot e of an operand holds: the order
+// in which dequant8 produces the codes of BITS.
+template <int BITS>
+__device__ constexpr int slot_channel(int e) {
+  return BITS == 4 ? ((e & 1) << 2) + ((e >> 2) << 1) + ((e & 2) ? 0 : 1)  // 1 5 0 4 3 7 2 6
+         : BITS == 2 ? ((e & 1) << 2) + (e >> 1)                            // 0 4 1 5 2 6 3 7
+                     : e;
+}
+template <int BITS>
+constexpr int kLaneBytes = BITS == 3 ? 64 : 8 * BITS;  // code bytes of 64 channels (3-bit codes are raw int8)
+
+// Code bytes of one lane's 64 channels.
+template <int BITS>
+struct Codes {
+  u32x4 w[kLaneBytes<BITS> / 16];
+};
+
+// The codes of 8 channels (group ks of the lane's 64) as four fp16 pairs, exact.
+template <int BITS>
+__device__ __forceinline__ void codes8(const Codes<BITS>& cd, int ks, f16x2 (&c)[4]) {
+  if constexpr (BITS == 4) {
+    // nibble -> mantissa bits 4..7 of 64.0 with its top bit flipped: 72 + c
+    const uint32_t w = cd.w[ks >> 2][ks & 3];
+    const uint32_t o[4] = {((w << 4) & 0x00F000F0u) ^ 0x54805480u, (w & 0x00F000F0u) ^ 0x54805480u,
+                           ((w >> 4) & 0x00F000F0u) ^ 0x54805480u, ((w >> 8) & 0x00F000F0u) ^ 0x54805480u};
+    const f16x2 k72 = {static_cast<_Float16>(72.0f), static_cast<_Float16>(72.0f)};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c[j] = __builtin_bit_cast(f16x2, o[j]) - k72;
+  } else if constexpr (BITS == 2) {
+    // two code bytes, one per half; a code -> mantissa bits 8..9 of 4.0 with its top bit flipped: 6 + c
+    const uint32_t d = cd.w[0][ks >> 1];
+    const uint32_t t = __builtin_amdgcn_perm(d, d, (ks & 1) ? 0x0C030C02u : 0x0C010C00u);
+    const f16x2 k6 = {static_cast<_Float16>(6.0f), static_cast<_Float16>(6.0f)};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      c[j] = __builtin_bit_cast(f16x2, ((t << (2 + 2 * j)) & 0x03000300u) ^ 0x46004600u) - k6;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t d = cd.w[ks >> 1][2 * (ks & 1) + (j >> 1)] >> (16 * (j & 1));
+      c[j] = f16x2{static_cast<_Float16>(static_cast<float>(static_cast<int8_t>(d & 0xFFu))),
+                   static_cast<_Float16>(static_cast<float>(static_cast<int8_t>((d >> 8) & 0xFFu)))};
+    }
+  }
+}
+
+// dtype(code * scale) for the pairs of codes8; s: the scales of each pair
+// (16-bit patterns, low half first).  fp16: one packed multiply, rounded once.
+// bf16: the product of a small integer and 8 bits is exact in fp32.
+template <bool BF>
+__device__ __forceinline__ uint32_t scaled(f16x2 c, uint32_t s) {
+#pragma clang fp contract(off)
+  if constexpr (BF)
+    return pack_bf16(static_cast<float>(c.x) * __uint_as_float(s << 16),
+                     static_cast<float>(c.y) * __uint_as_float(s & 0xFFFF0000u));
+  else
+    return __builtin_bit_cast(uint32_t, c * __builtin_bit_cast(f16x2, s));
+}
+
+template <bool BF>
+__device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
+  if constexpr (BF)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+// A scale whose products with the codes may not be finite: |s| >= 8192 (fp16) or
+// 2^125 (bf16), inf and NaN among them.
+template <bool BF>
+__device__ __forceinline__ bool big_scale(uint32_t bits) { return (bits & 0x7FFFu) >= (BF ? 0x7E00u : 0x7000u); }
+
+// The 16-bit values that are inf or NaN replaced by 0.
+template <bool BF>
+__device__ __forceinline__ u32x4 finite_only(u32x4 v) {
+  constexpr uint32_t kExp = BF ? 0x7F80u : 0x7C00u;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if ((v[j] & kExp) == kExp) v[j] &= 0xFFFF0000u;
+    if (((v[j] >> 16) & kExp) == kExp) v[j] &= 0x0000FFFFu;
+  }
+  return v;
+}
+
+// Work item `it` of a wave: 32 NT rows of one (b, h) slice (per-channel scales),
+// or of the flattened rows (per-token scales: one slice).
+template <int BITS, bool BF, int NT, bool TOKEN>
+__global__ __launch_bounds__(kThreads) void rotdq_kernel(const uint8_t* __restrict__ packed,
+                                                         const uint16_t* __restrict__ scale, int64_t S,
+                                                         uint32_t blocks, uint32_t items, const float* __restrict__ R,
+                                                         uint16_t* __restrict__ out) {
+  constexpr int NP = BF ? 3 : 2;  // pieces of R
+  constexpr int LB = kLaneBytes<BITS>;
+  constexpr int RB = 2 * LB;  // bytes per packed row
+  constexpr int kWaveRows = 32 * NT;
+  __shared__ __attribute__((aligned(16))) uint16_t rt[NP][kD][kRPitch];
+  __shared__ __attribute__((aligned(16))) uint8_t stage[kWaves][kWaveRows * kStagePitch];
+  __shared__ float red[kWaves];
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // ---- R^T in pieces into LDS: a thread turns the 2 x 4 blocks of two input
+  // channels in neighbouring slots and four output channels, one dword per
+  // output channel and piece.  A wave's 16 slot pairs x 4 channel quads put
+  // two lanes on a bank (2-byte writes of one row at a time put eight) ----
+  float unscale = 1.0f;
+  {
+    constexpr int kBlocks = kD / 2 * kD / 4 / kThreads;  // 2 x 4 blocks per thread
+    float4 ra[kBlocks], rb[kBlocks];
+    const int pair = tid & 15, quad = (tid >> 4) & 3, rest = tid >> 6;
+    float mx = 0.0f;
+    auto abs4 = [](const float4& v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); };
+    // block i: slots 2 pp, 2 pp + 1 (pp = pair + 16 (k & 3)), output channels 4 (quad + 4 (k >> 2)) ..+ 3
+#pragma unroll
+    for (int i = 0; i < kBlocks; ++i) {
+      const int k = rest + i * kWaves, pp = pair + 16 * (k & 3), e = 2 * (pp & 3), j0 = 4 * (quad + 4 * (k >> 2));
+      const float* src = R + (8 * (pp >> 2)) * kD + j0;
+      ra[i] = *reinterpret_cast<const float4*>(src + slot_channel<BITS>(e) * kD);
+      rb[i] = *reinterpret_cast<const float4*>(src + slot_channel<BITS>(e + 1) * kD);
+      mx = fmaxf(mx, fmaxf(abs4(ra[i]), abs4(rb[i])));
+    }
+    float scale_r = 1.0f;
+    if constexpr (!BF) {
+      mx = group_max<64>(mx);
+      if (lane == 0) red[wave] = mx;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) mx = fmaxf(mx, red[w]);
+      // 2^e with max|R| 2^e in [512, 1024); an orthogonal R's largest entry is at most 1
+      const int e = (mx > 0.0f && mx < INFINITY) ? 9 - ilogbf(mx) : 0;
+      const int ec = e < -60 ? -60 : (e > 60 ? 60 : e);
+      scale_r = ldexpf(1.0f, ec);
+      unscale = ldexpf(1.0f, -ec);
+    }
+#pragma unroll
+    for (int i = 0; i < kBlocks; ++i) {
+      const int k = rest + i * kWaves, pp = pair + 16 * (k & 3), j0 = 4 * (quad + 4 * (k >> 2));
+      const float fa[4] = {ra[i].x, ra[i].y, ra[i].z, ra[i].w}, fb[4] = {rb[i].x, rb[i].y, rb[i].z, rb[i].w};
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        // output channel 32 mt + 16 h' + 4 a + b sits in A row 32 mt + 8 a + 4 h' + b
+        const int j = j0 + jj, row = (j & ~31) | (((j >> 2) & 3) << 3) | (((j >> 4) & 1) << 2) | (j & 3);
+        float a = fa[jj] * scale_r, b = fb[jj] * scale_r;
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          const uint16_t pa = f2w<BF>(a), pb = f2w<BF>(b);
+          *reinterpret_cast<uint32_t*>(&rt[q][row][2 * pp]) = pa | (static_cast<uint32_t>(pb) << 16);
+          a -= w2f<BF>(pa);
+          b -= w2f<BF>(pb);
+        }
+      }
+    }
+  }
+  __syncthreads();
+
+  auto rows_of = [&](uint32_t it, int64_t& slice, int64_t& r0) {  // the wave's first row of item it
+    const uint32_t sl = TOKEN ? 0u : it / blocks;
+    slice = sl;
+    r0 = static_cast<int64_t>(it - sl * blocks) * kWaveRows;
+  };
+  auto load = [&](uint32_t it, Codes<BITS> (&cd)[NT], uint32_t (&ts)[NT]) {
+    int64_t slice, r0;
+    rows_of(it, slice, r0);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int64_t rr = r0 + 32 * t + n;
+      const int64_t row = slice * S + (rr < S ? rr : S - 1);  // rows past the slice: its last row, never stored
+      const u32x4* src = reinterpret_cast<const u32x4*>(packed + row * RB + h * LB);
+#pragma unroll
+      for (int k = 0; k < LB / 16; ++k) cd[t].w[k] = src[k];
+      ts[t] = TOKEN ? scale[row] : 0u;
+    }
+  };
+
+  // neighbouring items go to different workgroups, so a few of them spread over the CUs
+  for (uint32_t it = wave * gridDim.x + blockIdx.x; it < items; it += kWaves * gridDim.x) {
+    Codes<BITS> cd[NT];
+    uint32_t ts[NT];
+    load(it, cd, ts);
+    __asm__ volatile("" ::: "memory");  // keep the R fragment reads inside the loop
+    int64_t slice, r0;
+    rows_of(it, slice, r0);
+    u32x4 x[NT][8];
+    bool big = false;
+    if constexpr (TOKEN) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const uint32_t s2 = ts[t] | (ts[t] << 16);
+        big |= big_scale<BF>(ts[t]);
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+          f16x2 c[4];
+          codes8<BITS>(cd[t], ks, c);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) x[t][ks][j] = scaled<BF>(c[j], s2);
+        }
+      }
+    }
+    else {
+      const u32x4* sp = reinterpret_cast<const u32x4*>(scale + slice * kD + 64 * h);
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks) {
+        const u32x4 sw = sp[ks];
+        uint32_t sv[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          sv[j] = (sw[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
+          big |= big_scale<BF>(sv[j]);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          f16x2 c[4];
+          codes8<BITS>(cd[t], ks, c);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            x[t][ks][j] = scaled<BF>(c[j], sv[slot_channel<BITS>(2 * j)] | (sv[slot_channel<BITS>(2 * j + 1)] << 16));
+        }
+      }
+    }
+    // inf times a piece of R of either sign would give NaN where the whole
+    // entry gives inf: rows that may hold one multiply the lower pieces by
+    // their finite values only
+    const bool any_big = __builtin_amdgcn_ballot_w64(big) != 0;
+#pragma unroll 1
+    for (int mt = 0; mt < 4; ++mt) {
+      f32x16 acc[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = f32x16{};
+      if (__builtin_expect(!any_big, 1)) {
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks)
+#pragma unroll
+          for (int q = 0; q < NP; ++q) {
+            const u32x4 a = *reinterpret_cast<const u32x4*>(&rt[q][32 * mt + n][64 * h + 8 * ks]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[t] = mfma<BF>(a, x[t][ks], acc[t]);
+          }
+      } else {
+#pragma unroll 1
+        for (int q = 0; q < NP; ++q) {
+#pragma unroll
+          for (int ks = 0; ks < 8; ++ks) {
+            const u32x4 a = *reinterpret_cast<const u32x4*>(&rt[q][32 * mt + n][64 * h + 8 * ks]);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+              u32x4 xv = x[t][ks];
+              __asm__ volatile("" : "+v"(xv));  // computed here, in this rare branch, not ahead of the loop
+              acc[t] = mfma<BF>(a, q == 0 ? xv : finite_only<BF>(xv), acc[t]);
+            }
+          }
+        }
+      }
+      // lane (n, h): channels 32 mt + 16 h ..+ 15 of row n of each tile -> the wave's stage
+      uint8_t* const st = &stage[wave][0];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        u32x4 o[2];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float a = acc[t][2 * j] * unscale, b = acc[t][2 * j + 1] * unscale;
+          o[j >> 2][j & 3] = BF ? pack_bf16(a, b) : static_cast<uint32_t>(f2h(a)) | (static_cast<uint32_t>(f2h(b)) << 16);
+        }
+        u32x4* dst = reinterpret_cast<u32x4*>(st + (32 * t + n) * kStagePitch + 32 * h);
+        dst[0] = o[0];
+        dst[1] = o[1];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      // out in whole 64-byte row segments
+#pragma unroll
+      for (int k = 0; k < 2 * NT; ++k) {
+        const int rr = 16 * k + (lane >> 2);
+        const u32x4 v = *reinterpret_cast<const u32x4*>(st + rr * kStagePitch + 16 * (lane & 3));
+        if (r0 + rr < S)
+          *reinterpret_cast<u32x4*>(out + (slice * S + r0 + rr) * kD + 32 * mt + 8 * (lane & 3)) = v;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  }
+}
+
+template <int BITS, bool BF, bool TOKEN>
+void launch(const uint8_t* packed, const uint16_t* scale, int64_t BH, int64_t S, const float* R, uint16_t* out,
+            hipStream_t st) {
+  const int64_t slices = TOKEN ? 1 : BH, rows = TOKEN ? BH * S : S;
+  const int cus = num_cus();
+  // two row tiles per wave once that still gives every wave of the grid one
+  // (fp16 only: bf16's third piece of R leaves no LDS for the stage, raw int8
+  // 3-bit codes no registers)
+  constexpr int NT = BITS != 3 && !BF ? 2 : 1;
+  const int64_t waves = static_cast<int64_t>(cus) * kWaves;
+  const int nt = slices * cdiv(rows, 32 * NT) >= waves ? NT : 1;
+  const uint32_t blocks = static_cast<uint32_t>(cdiv(rows, 32 * nt)), items = static_cast<uint32_t>(slices * blocks);
+  const dim3 grid(items < static_cast<uint32_t>(cus) ? items : cus);
+  if (NT == 2 && nt == 2)
+    hipLaunchKernelGGL((rotdq_kernel<BITS, BF, NT, TOKEN>), grid, dim3(kThreads), 0, st, packed, scale, rows, blocks, items, R, out);
+  else
+    hipLaunchKernelGGL((rotdq_kernel<BITS, BF, 1, TOKEN>), grid, dim3(kThreads), 0, st, packed, scale, rows, blocks, items, R, out);
+}
+
+}  // namespace
+}  // namespace fade
+
+using namespace fade;
+
+FADE_API int fade_rotate_dequant(const void* packed, const void* scale, int32_t dtype, int32_t bits, int32_t axis,
+                                 int64_t B, int64_t H, int64_t S, int64_t D, const float* R, void* out, void* stream) {
+  const char* fn = "fade_rotate_dequant";
+  if (B < 0 || H < 0 || S < 0) return einval("%s: negative dimension", fn);
+  if (D != kD) return einval("%s: head_dim must be %d, got %lld", fn, kD, (long long)D);
+  if (bits != 2 && bits != 3 && bits != 4) return einval("%s: bits must be 2, 3 or 4, got %d", fn, bits);
+  if (axis != FADE_AXIS_TOKEN && axis != FADE_AXIS_CHANNEL) return einval("%s: bad axis %d", fn, axis);
+  if (dtype != FADE_DTYPE_F16 && dtype != FADE_DTYPE_BF16)
+    return einval("%s: dtype must be FADE_DTYPE_F16 or FADE_DTYPE_BF16, got %d", fn, dtype);
+  if (B * H * S == 0) return FADE_OK;
+  if (B * H * S > (int64_t{1} << 38)) return einval("%s: shape too large", fn);  // work items are 32-bit
+  if (packed == nullptr || scale == nullptr || R == nullptr || out == nullptr) return einval("%s: null pointer", fn);
+  if (((reinterpret_cast<uintptr_t>(packed) | reinterpret_cast<uintptr_t>(R) | reinterpret_cast<uintptr_t>(out)) & 15) ||
+      (reinterpret_cast<uintptr_t>(scale) & (axis == FADE_AXIS_CHANNEL ? 15 : 1)))
+    return einval("%s: packed, R, out and a per-channel scale must be 16-byte aligned", fn);
+  const uint8_t* pk = static_cast<const uint8_t*>(packed);
+  const uint16_t* sc = static_cast<const uint16_t*>(scale);
+  uint16_t* o = static_cast<uint16_t*>(out);
+  hipStream_t st = as_stream(stream);
+  const bool bf = dtype == FADE_DTYPE_BF16, token = axis == FADE_AXIS_TOKEN;
+#define FADE_ROTDQ(BITS)                                                          \
+  if (bf && token) launch<BITS, true, true>(pk, sc, B * H, S, R, o, st);          \
+  else if (bf) launch<BITS, true, false>(pk, sc, B * H, S, R, o, st);             \
+  else if (token) launch<BITS, false, true>(pk, sc, B * H, S, R, o, st);          \
+  else launch<BITS, false, false>(pk, sc, B * H, S, R, o, st);
+  if (bits == 4) { FADE_ROTDQ(4) }
+  else if (bits == 2) { FADE_ROTDQ(2) }
+  else { FADE_ROTDQ(3) }
+#undef FADE_ROTDQ
+  return check_launch(fn);
+}

@@ -381,18 +381,6 @@ __global__ __launch_bounds__(kThreads) void rotq_channel_kernel(const uint16_t* 
   }
 }
 
-int num_cus() {
-  static int cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
-}
-
 // S-blocking of the per-channel passes: about one block per CU in all (a
 // block holds most of a CU's LDS), at least 256 rows per block.
 void rotq_blocking(int64_t BH, int64_t S, int64_t* nsb, int64_t* rows_per_block) {

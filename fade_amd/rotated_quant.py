@@ -8,9 +8,11 @@ bit-pack); x_rot never reaches HBM.  Other shapes and dtypes take the two-step
 path: an fp32 GEMM through torch, then ``fade_quant_rotated``, which is
 bit-exact given ``x_rot`` (``quant_rotated_given``); bfloat16 and float32
 inputs get their scale in their own dtype (one rounding of the fp32
-``absmax / qmax``, as the reference's ``scale.to(k.dtype)``).  Dequantize is
-``dtype(code * scale)`` in ``fade_dequant_sym`` followed by the fp32 ``@ R``
-GEMM.
+``absmax / qmax``, as the reference's ``scale.to(k.dtype)``).  Dequantize to
+fp16 or bf16 at head_dim 128 is one kernel, ``fade_rotate_dequant``
+(``dtype(code * scale)`` in registers, then ``@ R`` on the matrix cores at
+fp32-GEMM accuracy); elsewhere ``dtype(code * scale)`` in ``fade_dequant_sym``
+followed by the fp32 ``@ R`` GEMM.
 """
 
 from __future__ import annotations
@@ -21,7 +23,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from .quant import _pack_codes, _unpack_codes, dequant_sym
+from .quant import _pack_codes, _scale_axis, _unpack_codes, dequant_sym
 
 DEFAULT_SEED: int = 42
 EPS: float = 1e-8
@@ -151,7 +153,40 @@ def rotated_dequant_rot(packed: Tensor, scale: Tensor, bits: int, dtype: torch.d
     return dequant_sym(packed, scale, bits, dtype)
 
 
+def _dequant_fused_ok(packed: Tensor, R: Tensor, bits: int, dtype) -> bool:
+    """Whether ``fade_rotate_dequant`` takes this call: its output types and head_dim, rows it
+    can read 16 bytes at a time, and no gradient wanted of R (the kernel records none)."""
+    return (
+        dtype in (torch.float16, torch.bfloat16)
+        and bits in _BIT_PARAMS
+        and packed.dim() == 4
+        and packed.is_cuda
+        and packed.shape[-1] == (128 if bits == 3 else 16 * bits)
+        and tuple(R.shape) == (128, 128)
+        and not (R.requires_grad and torch.is_grad_enabled())
+    )
+
+
+def _rotated_dequant_fused(packed: Tensor, scale: Tensor, R: Tensor, bits: int, dtype) -> Tensor:
+    _lib.require_gpu(packed, scale, op="dequant")
+    axis = _scale_axis(packed, scale)
+    B, H, S = packed.shape[:3]
+    out = torch.empty(B, H, S, 128, dtype=dtype, device=packed.device)
+    if out.numel() == 0:
+        return out
+    packed, scale = packed.contiguous(), scale.to(dtype).contiguous()
+    R = R.to(packed.device, dtype=torch.float32).contiguous()
+    packed, scale, R = (t.clone() if t.data_ptr() % 16 else t for t in (packed, scale, R))
+    _lib.call(
+        "fade_rotate_dequant", packed.data_ptr(), scale.data_ptr(), _lib.DTYPE_CODES[dtype], bits, axis, B, H, S, 128,
+        R.data_ptr(), out.data_ptr(), _lib.stream_of(packed),
+    )
+    return out
+
+
 def _rotated_dequant(packed, scale, R, bits, dtype):
+    if _dequant_fused_ok(packed, R, bits, dtype):
+        return _rotated_dequant_fused(packed, scale, R, bits, dtype)
     # the rotation back runs as an fp32 GEMM for every dtype (the reference's
     # CPU path; on CUDA it multiplies bf16 in bf16)
     x_rot = rotated_dequant_rot(packed, scale, bits, dtype if dtype in _lib.DTYPE_CODES else torch.float32)

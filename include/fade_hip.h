@@ -157,6 +157,15 @@ int fade_rotate_quant(const void* x_f16, int64_t B, int64_t H, int64_t S, int64_
                       int64_t sh, int64_t ss, const float* R, int32_t bits, int32_t axis,
                       void* packed, void* scale_f16, void* workspace, int64_t workspace_bytes,
                       void* stream);
+/* Fused dequantize + rotate back (fade/rotated_quant.py:134-145, 176-187):
+ * out [B,H,S,128] = dtype((dtype(code * scale)) @ R) with R fp32 [128,128]
+ * row-major on the device, on 16-bit matrix cores with R split into pieces
+ * (fp32-GEMM accuracy).  scale and out are of dtype (FADE_DTYPE_F16 or
+ * FADE_DTYPE_BF16); packed, R and out are contiguous and 16-byte aligned;
+ * scale is [B,H,1,128] (axis CHANNEL, 16-byte aligned) or [B,H,S,1] (axis TOKEN). */
+int fade_rotate_dequant(const void* packed, const void* scale, int32_t dtype, int32_t bits, int32_t axis,
+                        int64_t B, int64_t H, int64_t S, int64_t D, const float* R, void* out,
+                        void* stream);
 
 /* ---------------- asymmetric per-token groups (build format, no reference
  * counterpart: BASELINE's "asymmetric group-32 scale/zero") ------------- */
