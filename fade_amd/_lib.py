@@ -194,6 +194,8 @@ _SIGNATURES: dict[str, list] = {
     "fade_reassign_plan": [_p, _i64, _i64, _i64, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p],
     "fade_reassign_gather": [ctypes.POINTER(ReassignArgs), _p],
     "fade_tiered_prefill_attn": [ctypes.POINTER(PrefillArgs), _p],
+    "fade_tiered_prefill_workspace_bytes": [ctypes.POINTER(PrefillArgs), _pi64],
+    "fade_tiered_prefill_attn_ws": [ctypes.POINTER(PrefillArgs), _p, _i64, _p],
 }
 _RESTYPES = {"fade_hip_last_error": ctypes.c_char_p}
 

@@ -112,6 +112,13 @@ struct PParams {
   int mask_mode;          // FADE_MASK_*: bottom-right over the chunk, top-left over the row, none
   int chunk_len;          // chunk keys (Sq under FADE_MASK_BOTTOM_RIGHT)
   int D;                  // head_dim: a multiple of 8 up to the instance's capacity (packed middle: of 32)
+  // key splits (SPLIT instances): workgroup z = splits * (dispatched row) + split
+  // walks tiles split_tiles * split ..+ split_tiles - 1 of its row's sequence and leaves
+  // its unnormalized sums: part_o[row][split][D] and (max, sum) part_ml[row][split],
+  // row = (b * Hq + query head) * Sq + query
+  int splits, split_tiles;
+  float* part_o;
+  float2* part_ml;
 };
 
 // Eight two's-complement nibbles (one dword of packed codes, high nibble =
@@ -170,7 +177,7 @@ __host__ __device__ constexpr int swap23(int k) { return (k & ~12) | ((k & 4) <<
 // DP = 256 runs NQB = 1 at one wave per SIMD: its O accumulators alone take 128
 // registers per lane, and its LDS (two 33 KB K and two 36 KB V^T buffers) one
 // workgroup per CU.
-template <int DP, int NQB, bool BF>
+template <int DP, int NQB, bool BF, bool SPLIT>
 __global__ __launch_bounds__(kThreads * NQB) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<DP>, kWavesPerEu<DP>)))
 void prefill_kernel(PParams p) {
   static_assert(DP <= 128 || NQB == 1, "head_dim 256 runs one query block per workgroup");
@@ -191,9 +198,10 @@ void prefill_kernel(PParams p) {
   const int qb = blockIdx.x / p.passes;
   const int h0 = 4 * (blockIdx.x - qb * p.passes);  // first query head (within the group) of this workgroup
   const int64_t kvh = blockIdx.y;
-  int64_t b = blockIdx.z;
+  const int zrow = SPLIT ? blockIdx.z / p.splits : blockIdx.z, split = SPLIT ? blockIdx.z - zrow * p.splits : 0;
+  int64_t b = zrow;
   if (p.order) {
-    const int o = __builtin_amdgcn_readfirstlane(p.order[blockIdx.z]);
+    const int o = __builtin_amdgcn_readfirstlane(p.order[zrow]);
     b = o < 0 ? 0 : (o >= p.B ? p.B - 1 : o);
   }
   const int tid = threadIdx.x, lane = tid & 63;
@@ -238,6 +246,9 @@ void prefill_kernel(PParams p) {
     };
     n_tiles = upto(nts, 0) + upto(ntm, ns) + upto(ntr, ns + nm) + upto(ntc, ns + nm + nr);
   }
+  // this workgroup's tiles: all of them, or its split's
+  const int t0 = SPLIT ? split * p.split_tiles : 0;
+  const int t1 = SPLIT && t0 + p.split_tiles < n_tiles ? t0 + p.split_tiles : n_tiles;
   struct TileRef {
     int seg, base, cnt, gbase;  // segment (0 sink, 1 middle, 2 recent, 3 chunk), first key, keys,
                                 // first key's index in the row's sequence
@@ -641,18 +652,37 @@ void prefill_kernel(PParams p) {
   };
 
   __syncthreads();  // segd
-  if (begin_tile(0, 0)) store_mid(0);
-  __syncthreads();
-  for (int t = 0; t < n_tiles; ++t) {
-    const int buf = t & 1;
+  if (!SPLIT || t0 < t1) {  // (a split past the row's tiles leaves empty sums)
+    if (begin_tile(t0, 0)) store_mid(0);
+    __syncthreads();
+  }
+  for (int t = t0; t < t1; ++t) {
+    const int buf = (t - t0) & 1;
     // the next tile goes to the other buffer, last read by the previous tile's compute
-    const bool mid_next = t + 1 < n_tiles && begin_tile(t + 1, buf ^ 1);
+    const bool mid_next = t + 1 < t1 && begin_tile(t + 1, buf ^ 1);
     if (active) compute(t, buf);
     if (mid_next) store_mid(buf ^ 1);
     __syncthreads();
   }
 
   if (!active) return;
+  if constexpr (SPLIT) {  // ---- the split's unnormalized sums ----
+    const float lt = l_run + __shfl_xor(l_run, 32, 64);
+    const int64_t row0 = (b * p.Hq + hq) * Sq;
+    if (h == 0 && j0 + n32 < Sq) p.part_ml[(row0 + j0 + n32) * p.splits + split] = make_float2(m_run, lt);
+    if (t0 >= t1) return;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int j = j0 + 8 * (i >> 2) + 4 * h + (i & 3);
+      if (j < Sq) {
+        float* orow = p.part_o + ((row0 + j) * p.splits + split) * Dr;
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb)
+          if (32 * cb + n32 < Dr) orow[32 * cb + n32] = acc[cb][i];
+      }
+    }
+    return;
+  }
   // ---- normalize and store: 1 / l of each query row through LDS ----
   {
     const float lt = l_run + __shfl_xor(l_run, 32, 64);
@@ -673,6 +703,35 @@ void prefill_kernel(PParams p) {
       }
     }
   }
+}
+
+// The splits' sums of a query row merged in fp32 and in split order, normalized
+// and stored: D / 4 threads per row, four channels each.
+template <bool BF>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PParams p, int64_t rows) {
+  const int tpr = p.D / 4, rpb = 256 / tpr;
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * rpb + threadIdx.x / tpr;
+  const int c = 4 * (threadIdx.x % tpr);
+  if (threadIdx.x >= static_cast<unsigned>(rpb * tpr) || row >= rows) return;
+  const float2* ml = p.part_ml + row * p.splits;
+  float m = kNegBig;
+  for (int s = 0; s < p.splits; ++s) m = fmaxf(m, ml[s].x);
+  float l = 0.0f;
+  f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+  for (int s = 0; s < p.splits; ++s) {
+    const float2 w = ml[s];
+    f32x4 a = *reinterpret_cast<const f32x4*>(p.part_o + (row * p.splits + s) * p.D + c);
+    const float f = __builtin_amdgcn_exp2f((w.x - m) * p.scale_log2);
+    if (w.y == 0.0f) a = f32x4{};  // no visible key in this split: its part_o may not have been written
+    l += w.y * f;
+    o += a * f;
+  }
+  const float inv = 1.0f / l;
+  const int64_t j = row % p.Sq, bh = row / p.Sq;
+  uint16_t* dst = p.out + (bh / p.Hq) * p.o_sb + (bh % p.Hq) * p.o_sh + j * p.o_ss + c;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) dst[i] = f2w<BF>(o[i] * inv);
 }
 
 bool aligned16(const void* x) { return (reinterpret_cast<uintptr_t>(x) & 15) == 0; }
@@ -698,7 +757,10 @@ Tier tier_of(const fade_fp16_tier& t) {
 using namespace fade;
 using namespace fade::prefill;
 
-FADE_API int fade_tiered_prefill_attn(const fade_prefill_args* a, void* stream) {
+namespace {
+
+// Checks the arguments and fills the kernel's parameters (no split).
+int prefill_params(const fade_prefill_args* a, PParams& p) {
   if (a == nullptr) return einval("fade_tiered_prefill_attn: null args");
   if (a->D < 8 || a->D > 256 || a->D % 8 != 0)
     return einval("fade_tiered_prefill_attn: head_dim must be a multiple of 8 in [8, 256], got %lld", (long long)a->D);
@@ -740,7 +802,7 @@ FADE_API int fade_tiered_prefill_attn(const fade_prefill_args* a, void* stream) 
     if (m.pages != nullptr && (m.page_stride != 0 || m.pages_per_row * kKT < m.len))
       return einval("fade_tiered_prefill_attn: a paged middle tier needs separate pools and pages_per_row * 64 >= len");
   }
-  PParams p{};
+  p = PParams{};
   p.B = a->B;
   p.Hq = a->Hq;
   p.Hkv = a->Hkv;
@@ -748,7 +810,6 @@ FADE_API int fade_tiered_prefill_attn(const fade_prefill_args* a, void* stream) 
   p.G = static_cast<int>(a->Hq / a->Hkv);
   p.passes = (p.G + 3) / 4;
   p.hpw = p.G >= 3 ? 4 : p.G;
-  const int qpg = 4 / p.hpw;  // query blocks per group of 4 waves
   p.q = static_cast<const uint16_t*>(a->q);
   p.q_sb = a->q_sb; p.q_sh = a->q_sh; p.q_ss = a->q_ss;
   p.out = static_cast<uint16_t*>(a->out);
@@ -773,23 +834,114 @@ FADE_API int fade_tiered_prefill_attn(const fade_prefill_args* a, void* stream) 
   p.mask_mode = a->mask_mode;
   p.chunk_len = static_cast<int>(a->chunk.len);
   p.D = static_cast<int>(a->D);
-  // two groups of 4 waves once one group's query blocks do not cover the chunk
-  // (one at head_dim > 128)
-  const int nqb = a->Sq > kQB * qpg && a->D <= 128 ? 2 : 1;
-  const dim3 grid(static_cast<unsigned>(cdiv(a->Sq, kQB * nqb * qpg) * p.passes), static_cast<unsigned>(a->Hkv),
-                  static_cast<unsigned>(a->B));
-  const bool bf = a->dtype == FADE_DTYPE_BF16;
-#define FADE_PREFILL_LAUNCH(DD)                                                                                        \
-  if (bf && nqb == 2) hipLaunchKernelGGL((prefill_kernel<DD, 2, true>), grid, dim3(2 * kThreads), 0, as_stream(stream), p); \
-  else if (bf) hipLaunchKernelGGL((prefill_kernel<DD, 1, true>), grid, dim3(kThreads), 0, as_stream(stream), p);           \
-  else if (nqb == 2) hipLaunchKernelGGL((prefill_kernel<DD, 2, false>), grid, dim3(2 * kThreads), 0, as_stream(stream), p); \
-  else hipLaunchKernelGGL((prefill_kernel<DD, 1, false>), grid, dim3(kThreads), 0, as_stream(stream), p);
+  return FADE_OK;
+}
+
+// Query blocks of 32 per workgroup group (4 waves), and groups per workgroup:
+// two once one group's query blocks do not cover the chunk (one at head_dim > 128).
+int query_blocks(const PParams& p) { return 4 / p.hpw; }
+int groups(const PParams& p) { return p.Sq > kQB * query_blocks(p) && p.D <= 128 ? 2 : 1; }
+
+// Key splits of a call, from the sizes the host knows (the padded capacities).
+// Unsplit, a workgroup walks its row's whole sequence, and a call of few (query
+// block, kv head, row) triples leaves most CUs idle.  Splits are taken while
+// all workgroups run at once: past that a second round of them repeats the
+// prologue and moves more partial sums than the balance gains (12 rows of 4000
+// keys, 128 queries, 192 workgroups: 153 us unsplit, 203 in four splits).
+// Measured, unsplit -> split: 2 rows of 2999 + 333 keys at head_dim 64, 14/2
+// heads 111 -> 36 us (5 splits); one row of 4096 keys, 128 queries, 32/8 heads
+// 151 -> 35; 32 queries over 16000 keys 468 -> 35; 17 over 8000, 64/8 heads
+// 240 -> 32; 4 rows of 4000 at head_dim 256 280 -> 62.
+// The cost in tile times (about 2.2 us): the split's tiles, and kSums for
+// writing and merging the sums of a full round of workgroups (128 KB each at
+// head_dim 128), kMerge for the second launch.
+void plan_splits(PParams& p) {
+  constexpr int kSums = 3, kMerge = 1, kMost = 32, kLeast = 2;  // kLeast: fewest tiles of a split
+  const int64_t blocks = cdiv(p.Sq, kQB * groups(p) * query_blocks(p)) * p.passes * p.Hkv * p.B;
+  const int64_t tiles = cdiv(p.sink_cap, kKT) + cdiv(p.mid_cap, kKT) + cdiv(p.recent_cap, kKT) + cdiv(p.chunk_len, kKT);
+  // workgroups the chip holds at once: one of 8 waves per CU, two of 4 (one at head_dim > 128)
+  const int64_t slots = static_cast<int64_t>(num_cus()) * (groups(p) == 1 && p.D <= 128 ? 2 : 1);
+  int64_t best = tiles;
+  p.splits = 1;
+  p.split_tiles = static_cast<int>(tiles);
+  for (int s = 2; s <= kMost && s * kLeast <= tiles && blocks * s <= slots; ++s) {
+    const int64_t per = cdiv(tiles, s), n = cdiv(tiles, per);
+    const int64_t cost = per + kMerge + kSums * blocks * n / slots;
+    if (cost < best) {
+      best = cost;
+      p.splits = static_cast<int>(n);
+      p.split_tiles = static_cast<int>(per);
+    }
+  }
+}
+
+int64_t split_bytes(const PParams& p) {
+  return p.splits <= 1 ? 0 : p.B * p.Hq * p.Sq * p.splits * (p.D * 4 + static_cast<int64_t>(sizeof(float2)));
+}
+
+int prefill_launch(PParams& p, bool bf, void* stream) {
+  const int nqb = groups(p);
+  const dim3 grid(static_cast<unsigned>(cdiv(p.Sq, kQB * nqb * query_blocks(p)) * p.passes), static_cast<unsigned>(p.Hkv),
+                  static_cast<unsigned>(p.B * p.splits));
+  hipStream_t st = as_stream(stream);
+#define FADE_PREFILL_ONE(DD, NQ, BF)                                                                              \
+  if (p.splits > 1) hipLaunchKernelGGL((prefill_kernel<DD, NQ, BF, true>), grid, dim3(NQ * kThreads), 0, st, p);  \
+  else hipLaunchKernelGGL((prefill_kernel<DD, NQ, BF, false>), grid, dim3(NQ * kThreads), 0, st, p);
+#define FADE_PREFILL_LAUNCH(DD)                           \
+  if (bf && nqb == 2) { FADE_PREFILL_ONE(DD, 2, true) }   \
+  else if (bf) { FADE_PREFILL_ONE(DD, 1, true) }          \
+  else if (nqb == 2) { FADE_PREFILL_ONE(DD, 2, false) }   \
+  else { FADE_PREFILL_ONE(DD, 1, false) }
   // the smallest instance whose capacity covers the head_dim
-  if (a->D <= 32) { FADE_PREFILL_LAUNCH(32) }
-  else if (a->D <= 64) { FADE_PREFILL_LAUNCH(64) }
-  else if (a->D <= 128) { FADE_PREFILL_LAUNCH(128) }
-  else if (bf) hipLaunchKernelGGL((prefill_kernel<256, 1, true>), grid, dim3(kThreads), 0, as_stream(stream), p);
-  else hipLaunchKernelGGL((prefill_kernel<256, 1, false>), grid, dim3(kThreads), 0, as_stream(stream), p);
+  if (p.D <= 32) { FADE_PREFILL_LAUNCH(32) }
+  else if (p.D <= 64) { FADE_PREFILL_LAUNCH(64) }
+  else if (p.D <= 128) { FADE_PREFILL_LAUNCH(128) }
+  else if (bf) { FADE_PREFILL_ONE(256, 1, true) }
+  else { FADE_PREFILL_ONE(256, 1, false) }
 #undef FADE_PREFILL_LAUNCH
-  return check_launch("fade_tiered_prefill_attn");
+#undef FADE_PREFILL_ONE
+  const int rc = check_launch("fade_tiered_prefill_attn");
+  if (rc || p.splits <= 1) return rc;
+  const int64_t rows = p.B * p.Hq * p.Sq;
+  const dim3 mgrid(static_cast<unsigned>(cdiv(rows, 256 / (p.D / 4))));
+  if (bf) hipLaunchKernelGGL(prefill_merge_kernel<true>, mgrid, dim3(256), 0, st, p, rows);
+  else hipLaunchKernelGGL(prefill_merge_kernel<false>, mgrid, dim3(256), 0, st, p, rows);
+  return check_launch("fade_tiered_prefill_attn (merge)");
+}
+
+}  // namespace
+
+FADE_API int fade_tiered_prefill_workspace_bytes(const fade_prefill_args* a, int64_t* bytes) {
+  if (bytes == nullptr) return einval("fade_tiered_prefill_workspace_bytes: null output");
+  PParams p;
+  const int rc = prefill_params(a, p);
+  if (rc) return rc;
+  plan_splits(p);
+  *bytes = split_bytes(p);
+  return FADE_OK;
+}
+
+FADE_API int fade_tiered_prefill_attn_ws(const fade_prefill_args* a, void* workspace, int64_t workspace_bytes,
+                                         void* stream) {
+  PParams p;
+  const int rc = prefill_params(a, p);
+  if (rc) return rc;
+  plan_splits(p);
+  const int64_t need = split_bytes(p);
+  if (need > 0) {
+    if (workspace == nullptr || workspace_bytes < need || !aligned16(workspace))
+      return einval("fade_tiered_prefill_attn_ws: needs a 16-byte aligned workspace of %lld bytes", (long long)need);
+    const int64_t parts = p.B * p.Hq * p.Sq * p.splits;
+    p.part_o = static_cast<float*>(workspace);
+    p.part_ml = reinterpret_cast<float2*>(p.part_o + parts * p.D);
+  }
+  return prefill_launch(p, a->dtype == FADE_DTYPE_BF16, stream);
+}
+
+FADE_API int fade_tiered_prefill_attn(const fade_prefill_args* a, void* stream) {
+  PParams p;
+  const int rc = prefill_params(a, p);
+  if (rc) return rc;
+  p.splits = 1;
+  return prefill_launch(p, a->dtype == FADE_DTYPE_BF16, stream);
 }

@@ -23,7 +23,9 @@ _MASKS = {"bottom_right": _lib.MASK_BOTTOM_RIGHT, "top_left": _lib.MASK_TOP_LEFT
 
 
 class TieredPrefillPlan:
-    """Validated launch for fixed tensors; ``run()`` enqueues one kernel.
+    """Validated launch for fixed tensors; ``run()`` enqueues one kernel, or two where
+    the keys are split over workgroups (calls too small to fill the GPU; the plan keeps
+    the workspace of their partial sums, so runs of one plan must not overlap).
 
     Args:
         q: [B, Hq, Sq, D] fp16 or bf16 queries of the chunk; D a multiple of 8 up to 256.
@@ -118,12 +120,18 @@ class TieredPrefillPlan:
         a.dtype = dtc
         self.args = a
         self.out = out
-        self._fn = _lib.load().fade_tiered_prefill_attn
+        lib = _lib.load()
         self._argp = ctypes.byref(a)
+        nb = ctypes.c_int64(0)
+        lib.fade_tiered_prefill_workspace_bytes(self._argp, nb)  # (arguments it refuses are refused by run())
+        self.workspace = _lib.scratch(nb.value, q.device) if nb.value else None
+        self._fn = lib.fade_tiered_prefill_attn_ws
 
     def run(self, stream: int | None = None) -> Tensor:
         s = torch.cuda.current_stream(self.out.device).cuda_stream if stream is None else stream
-        _lib.check(self._fn(self._argp, s), "fade_tiered_prefill_attn")
+        ws = self.workspace
+        _lib.check(self._fn(self._argp, None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), s),
+                   "fade_tiered_prefill_attn")
         return self.out
 
 

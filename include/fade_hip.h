@@ -433,6 +433,14 @@ typedef struct fade_prefill_args {
 } fade_prefill_args;
 
 int fade_tiered_prefill_attn(const fade_prefill_args* args, void* stream);
+/* The same with a workspace for calls of few (query block, kv head, row)
+ * triples: their keys are then split over several workgroups, whose fp32 sums
+ * are merged in a fixed order by a second launch.  The query gives the bytes
+ * (0: no split, workspace may be NULL); 16-byte aligned, contents arbitrary,
+ * not shared by calls that may overlap. */
+int fade_tiered_prefill_workspace_bytes(const fade_prefill_args* args, int64_t* bytes);
+int fade_tiered_prefill_attn_ws(const fade_prefill_args* args, void* workspace, int64_t workspace_bytes,
+                                void* stream);
 
 #ifdef __cplusplus
 }
