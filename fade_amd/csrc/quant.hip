@@ -198,6 +198,35 @@ __device__ __forceinline__ uint32_t codes4_f16(const uint4& x, const uint4& inv)
   return __builtin_amdgcn_perm(uy, ty, 0x06040200u);
 }
 
+// The INT4 codes of eight bfloat16 values x times the inverse scales iv (fp32
+// values of bfloat16 numbers), packed as store_codes<4> packs them.  The
+// product is rounded to bfloat16 by the hardware pair conversion (nearest
+// even, as f2bf), clamped (integer bounds, so before the rounding to an integer
+// as well as after), and the sum with 1.5 * 2^23 rounds it half-to-even into
+// the low mantissa bits.  Equal to sym_code<MODE_BF16, -8, 7> for finite x and
+// finite iv (the product is then never NaN; an inf clamps).
+__device__ __forceinline__ uint32_t codes4_bf16(const uint4& x, const float* iv) {
+#pragma clang fp contract(off)
+  const uint32_t u[4] = {x.x, x.y, x.z, x.w};
+  uint32_t w = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t p = pack_bf16(__uint_as_float(u[j] << 16) * iv[2 * j], __uint_as_float(u[j] & 0xFFFF0000u) * iv[2 * j + 1]);
+    const float a = __builtin_amdgcn_fmed3f(__uint_as_float(p << 16), -8.0f, 7.0f) + 12582912.0f;
+    const float b = __builtin_amdgcn_fmed3f(__uint_as_float(p & 0xFFFF0000u), -8.0f, 7.0f) + 12582912.0f;
+    const uint32_t byte = ((__float_as_uint(a) & 0xFu) << 4) | (__float_as_uint(b) & 0xFu);
+    w |= byte << (8 * j);
+  }
+  return w;
+}
+// Eight bfloat16 values hold neither inf nor NaN.
+__device__ __forceinline__ bool finite8_bf16(const uint4& w) {
+  auto mag = [](uint32_t a) { return __builtin_bit_cast(u16x2, a & 0x7FFF7FFFu); };
+  const u16x2 t = __builtin_elementwise_max(__builtin_elementwise_max(mag(w.x), mag(w.y)),
+                                            __builtin_elementwise_max(mag(w.z), mag(w.w)));
+  return (t[0] > t[1] ? t[0] : t[1]) < 0x7F80u;
+}
+
 // The INT2 codes (clamped to [-2, 1]) of eight fp16 values, as eight int8
 // bytes: the same rounding as codes4_f16, clamped to [1534, 1537], whose low
 // byte is the code's two's complement.  Same validity as codes4_f16.
@@ -260,6 +289,7 @@ __global__ __launch_bounds__(kBlock) void quant_token_kernel(const InT* __restri
   const int c = threadIdx.x % LPR;
   const bool on = c * 8 < D;  // lanes past the row's D / 8 groups of 8 channels idle
   constexpr bool kPk = MODE == MODE_F16 && BITS == 4 && std::is_same<InT, uint16_t>::value;
+  constexpr bool kPkBf = MODE == MODE_BF16 && BITS == 4 && std::is_same<InT, Bf16>::value;
   for (int64_t r = static_cast<int64_t>(blockIdx.x) * RP + threadIdx.x / LPR; r < rows;
        r += static_cast<int64_t>(gridDim.x) * RP) {
     float v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -278,6 +308,17 @@ __global__ __launch_bounds__(kBlock) void quant_token_kernel(const InT* __restri
 #pragma unroll
         for (int j = 0; j < 8; ++j) a = absmax_nan(a, v[j]);
       }
+    } else if constexpr (kPkBf) {
+      if (on) raw = *reinterpret_cast<const uint4*>(src);
+      fin = finite8_bf16(raw);
+      const uint32_t u[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[2 * i] = __uint_as_float(u[i] << 16);
+        v[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a = absmax_nan(a, v[j]);
     } else {
       if (on) load8(src, v);
 #pragma unroll
@@ -295,6 +336,14 @@ __global__ __launch_bounds__(kBlock) void quant_token_kernel(const InT* __restri
         continue;
       }
       if (fin) f16x8_to_f32(raw, v);  // the scalar path below reads v
+    }
+    if constexpr (kPkBf) {
+      if (on && inv < INFINITY && fin) {  // (a NaN inv compares false)
+        const float iv[8] = {inv, inv, inv, inv, inv, inv, inv, inv};
+        *reinterpret_cast<uint32_t*>(packed + r * row_bytes + c * 4) = codes4_bf16(raw, iv);
+        if (c == 0) scale[r] = sc;
+        continue;
+      }
     }
     int code[8];
 #pragma unroll
@@ -351,7 +400,8 @@ __global__ __launch_bounds__(kBlock) void quant_channel_kernel(
   __shared__ float inv_s[DP];
   for (int d = threadIdx.x; d < D; d += kBlock) {
     float a = 0.0f;
-    for (int k = 0; k < nparts; ++k) a = absmax_nan(a, partial[(bh * nparts + k) * D + d]);
+#pragma unroll 16
+    for (int k = 0; k < nparts; ++k) a = absmax_nan(a, partial[(bh * nparts + k) * D + d]);  // loads in flight together
     float inv;
     typename ScaleOf<MODE>::T sc;
     sym_params<MODE, QRange<BITS>::hi>(a, inv, sc);
@@ -403,6 +453,260 @@ __global__ __launch_bounds__(kBlock) void quant_channel_kernel(
     for (int j = 0; j < 8; ++j) code[j] = sym_code<MODE, QRange<BITS>::lo, QRange<BITS>::hi>(v[j], iv[j]);
     store_codes<BITS>(packed + (bh * S + s) * row_bytes + c * lane_bytes<BITS>(), code);
   }
+}
+
+// Both passes in one for slices that several workgroups hold in registers: the
+// n workgroups of one (b, h) read their rows once, merge their column maxima
+// through memory, and quantize from registers.
+//
+// The two-pass form reads K twice, and at few (b, h) every workgroup of its second
+// pass first folds dozens of partial maxima.  Measured, both launches of a call
+// (two passes -> this): 16 x 8 x 8124 x 128 fp16 119.6 -> 67.9 us (332 MB, 4.9
+// TB/s), 4 x 8 x 32508 129.6 -> 76; 3 x 4 x 5003 bf16 32 -> 17 (then bound by the
+// host's launches); 1 x 8 x 30000 86 -> 23.
+//
+// A workgroup stores its maxima (bit patterns of magnitudes, which order as the
+// values, NaN above inf) with the patterns' free sign bits set, and reads the
+// others' until every dword has them: a dword carries its own mark, so no
+// order between stores is relied on.  Stores and loads are at system scope
+// (written through to memory and fetched from it); the area is zero at launch.
+// (Atomic maxima instead, one per channel and workgroup, took 314 us here.)
+//
+// The wait is bounded: after `polls` reads of a missing dword a workgroup stops
+// and computes its (b, h)'s maxima from x itself, the same values.  So the
+// kernel ends whatever order or number of its workgroups the chip runs at
+// once; with workgroups started in index order the n of a slice run together
+// and none gets there.
+template <typename InT>
+struct Row8 {  // eight elements of a row as loaded
+  uint4 w[sizeof(InT) / 2];
+};
+template <typename InT>
+__device__ __forceinline__ void row8_f32(const Row8<InT>& r, float* v) {
+  if constexpr (std::is_same<InT, uint16_t>::value) {
+    f16x8_to_f32(r.w[0], v);
+  } else if constexpr (std::is_same<InT, Bf16>::value) {
+    const uint32_t u[4] = {r.w[0].x, r.w[0].y, r.w[0].z, r.w[0].w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(u[i] << 16);
+      v[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      v[4 * i] = __uint_as_float(r.w[i].x);
+      v[4 * i + 1] = __uint_as_float(r.w[i].y);
+      v[4 * i + 2] = __uint_as_float(r.w[i].z);
+      v[4 * i + 3] = __uint_as_float(r.w[i].w);
+    }
+  }
+}
+// Running maxima of eight channels' magnitudes, as the bit patterns of InT
+// (16-bit types: two channels to a dword).
+template <typename InT>
+struct Mag8 {
+  uint32_t m[sizeof(InT) == 2 ? 4 : 8];
+};
+__device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+template <typename InT>
+__device__ __forceinline__ void mag8_add(Mag8<InT>& m, const Row8<InT>& r) {
+  if constexpr (sizeof(InT) == 2) {
+    const uint32_t u[4] = {r.w[0].x, r.w[0].y, r.w[0].z, r.w[0].w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m.m[i] = max_u16x2(m.m[i], u[i] & 0x7FFF7FFFu);
+  } else {
+    const uint32_t u[8] = {r.w[0].x, r.w[0].y, r.w[0].z, r.w[0].w, r.w[1].x, r.w[1].y, r.w[1].z, r.w[1].w};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m.m[i] = max(m.m[i], u[i] & 0x7FFFFFFFu);
+  }
+}
+template <typename InT>
+__device__ __forceinline__ float mag_f32(uint32_t bits) {
+  if constexpr (std::is_same<InT, uint16_t>::value) return h2f(static_cast<uint16_t>(bits));
+  else if constexpr (std::is_same<InT, Bf16>::value) return bf2f(static_cast<uint16_t>(bits));
+  else return __uint_as_float(bits);
+}
+
+// NT: non-temporal loads, for inputs that no cache holds.
+template <typename InT, int MODE, int BITS, int LPR, int NR, bool NT>
+__global__ __launch_bounds__(kBlock, 4) void quant_channel_once_kernel(
+    const InT* __restrict__ x, int D, int64_t H, int64_t S, int64_t sb, int64_t sh, int64_t ss, uint32_t* maxima,
+    int polls, uint8_t* __restrict__ packed, typename ScaleOf<MODE>::T* __restrict__ scale) {
+  constexpr int RP = kBlock / LPR;
+  constexpr int DP = LPR * 8;  // the instance's channel capacity (>= D)
+  constexpr int NM = sizeof(InT) == 2 ? 4 : 8;  // dwords of eight magnitudes
+  constexpr int NC = LPR * NM;                  // dwords of a row's magnitudes
+  constexpr int kW = kBlock / 64, kP = kBlock / NC;
+  constexpr uint32_t kMark = NM == 4 ? 0x80008000u : 0x80000000u;
+  const int row_bytes = (D / 8) * lane_bytes<BITS>();
+  const int64_t bh = blockIdx.y;
+  const int n = gridDim.x;
+  const int c = threadIdx.x % LPR, rs = threadIdx.x / LPR;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool on = c * 8 < D;  // lanes past the row's channels hold zeros
+  const int64_t s0 = static_cast<int64_t>(blockIdx.x) * (RP * NR) + rs;
+  const InT* base = x + (bh / H) * sb + (bh % H) * sh + (on ? c * 8 : 0);
+  auto load = [&](int64_t s) {
+    Row8<InT> r = {};
+    if (on && s < S) r = *reinterpret_cast<const Row8<InT>*>(base + s * ss);
+    return r;
+  };
+  auto max_of = [](uint32_t a, uint32_t b) { return NM == 4 ? max_u16x2(a, b) : max(a, b); };
+  __shared__ uint32_t red[kW][NC];
+  __shared__ uint32_t others[kP][NC];
+  __shared__ float inv_s[DP];
+  __shared__ int met;
+  const int col = threadIdx.x % NC, part = threadIdx.x / NC;  // dword of the row's magnitudes
+  // the threads' maxima -> the workgroup's, dword `col` in threads with part == 0
+  auto fold = [&](Mag8<InT> m) {
+#pragma unroll
+    for (int o = LPR; o < 64; o <<= 1)
+#pragma unroll
+      for (int i = 0; i < NM; ++i) m.m[i] = max_of(m.m[i], static_cast<uint32_t>(__shfl_xor(static_cast<int>(m.m[i]), o, 64)));
+    if (lane < LPR)
+#pragma unroll
+      for (int i = 0; i < NM; ++i) red[wave][lane * NM + i] = m.m[i];
+    __syncthreads();
+    uint32_t v = red[0][col];
+#pragma unroll
+    for (int w = 1; w < kW; ++w) v = max_of(v, red[w][col]);
+    return v;
+  };
+
+  Row8<InT> r[NR];
+  Mag8<InT> m = {};
+  // rows of the slice from this thread's first one on, at most the workgroup's
+  const int have = S - s0 < RP * NR ? static_cast<int>(S - s0) : RP * NR;
+  {
+    const InT* src = base + s0 * ss;
+#pragma unroll
+    for (int i = 0; i < NR; ++i, src += RP * ss) {
+      r[i] = Row8<InT>{};
+      if (!(on && i * RP < have)) continue;
+      if constexpr (NT) {
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+        for (unsigned k = 0; k < sizeof(Row8<InT>) / 16; ++k) {
+          const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src) + k);
+          r[i].w[k] = make_uint4(w.x, w.y, w.z, w.w);
+        }
+      } else {
+        r[i] = *reinterpret_cast<const Row8<InT>*>(src);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NR; ++i) mag8_add<InT>(m, r[i]);
+  if (threadIdx.x == 0) met = 1;
+  uint32_t top = fold(m);
+  if (n > 1) {
+    uint32_t* area = maxima + bh * n * NC + col;  // [workgroup][dword]
+    if (part == 0)
+      __hip_atomic_store(area + static_cast<int64_t>(blockIdx.x) * NC, top | kMark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    uint32_t all = top;
+    int left = polls;
+    for (int p0 = part; p0 < n; p0 += 8 * kP) {
+      uint32_t v[8];
+      for (;;) {
+        bool here = true;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int p = p0 + i * kP;
+          v[i] = p < n ? __hip_atomic_load(area + static_cast<int64_t>(p) * NC, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) : kMark;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) here = here && (v[i] & kMark) == kMark;
+        if (here || --left < 0) break;
+        __builtin_amdgcn_s_sleep(2);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) all = max_of(all, v[i] & ~kMark);
+    }
+    others[part][col] = all;
+    if (left < 0) met = 0;
+    __syncthreads();
+    if (met) {
+      top = others[0][col];
+#pragma unroll
+      for (int i = 1; i < kP; ++i) top = max_of(top, others[i][col]);
+    } else {
+      Mag8<InT> own = {};
+      for (int64_t s = rs; s < S; s += RP) mag8_add<InT>(own, load(s));
+      top = fold(own);
+    }
+  }
+  if (part == 0) {
+    constexpr int kPer = 8 / NM;  // channels per dword
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+      const int d = col * kPer + e;
+      if (d < D) {
+        float inv;
+        typename ScaleOf<MODE>::T sc;
+        sym_params<MODE, QRange<BITS>::hi>(mag_f32<InT>(NM == 4 ? (top >> (16 * e)) & 0x7FFFu : top), inv, sc);
+        inv_s[d] = inv;
+        if (blockIdx.x == 0) scale[bh * D + d] = sc;
+      }
+    }
+  }
+  __syncthreads();
+  if (!on) return;
+  float iv[8];
+  bool inv_pos = true, inv_fin = true;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    iv[j] = inv_s[c * 8 + j];
+    inv_pos = inv_pos && iv[j] > 0.0f && iv[j] < INFINITY;
+    inv_fin = inv_fin && fabsf(iv[j]) < INFINITY;
+  }
+  constexpr bool kPk = MODE == MODE_F16 && BITS == 4 && std::is_same<InT, uint16_t>::value;
+  constexpr bool kPkBf = MODE == MODE_BF16 && BITS == 4 && std::is_same<InT, Bf16>::value;
+  uint4 invv = make_uint4(0u, 0u, 0u, 0u);
+  if constexpr (kPk) {
+    uint32_t ivp[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      ivp[j] = static_cast<uint32_t>(f2h(iv[2 * j])) | (static_cast<uint32_t>(f2h(iv[2 * j + 1])) << 16);
+    invv = make_uint4(ivp[0], ivp[1], ivp[2], ivp[3]);
+  }
+  auto quantize = [&](const Row8<InT>& row, uint8_t* dst) {
+    if constexpr (kPk) {
+      if (inv_pos && finite8(row.w[0])) {
+        *reinterpret_cast<uint32_t*>(dst) = codes4_f16(row.w[0], invv);
+        return;
+      }
+    }
+    if constexpr (kPkBf) {
+      if (inv_fin && finite8_bf16(row.w[0])) {
+        *reinterpret_cast<uint32_t*>(dst) = codes4_bf16(row.w[0], iv);
+        return;
+      }
+    }
+    float v[8];
+    row8_f32<InT>(row, v);
+    int code[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) code[j] = sym_code<MODE, QRange<BITS>::lo, QRange<BITS>::hi>(v[j], iv[j]);
+    store_codes<BITS>(dst, code);
+  };
+  uint8_t* dst = packed + (bh * S + s0) * row_bytes + c * lane_bytes<BITS>();
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    if (i * RP < have) quantize(r[i], dst);
+    dst += RP * row_bytes;
+    // one row at a time: its temporaries in registers, not all rows'
+    __asm__ volatile("" : "+v"(dst) : : "memory");
+  }
+}
+
+// Zero words [0, n): the exchange area of quant_channel_once_kernel (a kernel, so
+// that a captured call stays a chain of kernels).
+__global__ __launch_bounds__(kBlock) void zero_words_kernel(uint32_t* p, int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (i < n) p[i] = 0u;
 }
 
 // ---------------------------------------------------------- dequant (sym)
@@ -834,6 +1138,46 @@ void channel_blocking(int64_t BH, int64_t S, int64_t* nsb, int64_t* rows_per_blo
   *nsb = cdiv(S, rpb) > 0 ? cdiv(S, rpb) : 1;
 }
 
+// Polls of quant_channel_once_kernel's wait, about 1 us each: far beyond the wait of
+// a slice whose workgroups run together (a few us).
+constexpr int kPolls = 256;
+// Inputs of at least half the 256 MB device cache are read with non-temporal loads
+// (266 MB: 71.7 -> 67.9 us; 61 MB, which the cache may hold: 23.0 -> 24.4).
+constexpr int64_t kStreamBytes = int64_t{1} << 27;
+// Workgroups of one (b, h) that may wait for each other: the chip holds at least
+// 512 of them (2 per CU), so the slices ahead of the last one are always complete.
+constexpr int64_t kMostWaiting = 128;
+
+// Rows per thread of the single-pass form and its workgroups per (b, h): 64
+// registers of row data, or 16 where that many per thread would leave CUs idle;
+// n = 0: the two-pass form.
+struct OncePlan {
+  bool big;
+  int64_t n, words;  // workgroups of a (b, h); dwords of all exchange areas
+};
+OncePlan once_plan(int64_t BH, int64_t S, int64_t D, int elem_bytes) {
+  const int lpr = D <= 32 ? 4 : D <= 64 ? 8 : D <= 128 ? 16 : 32;
+  const int64_t rp = kBlock / lpr, big = elem_bytes == 2 ? 16 : 8;
+  OncePlan pl{};
+  pl.big = BH * cdiv(S, rp * big) >= num_cus();
+  pl.n = cdiv(S, rp * (pl.big ? big : big / 4));
+  pl.words = BH * pl.n * lpr * (elem_bytes == 2 ? 4 : 8);
+  if (pl.n > kMostWaiting) pl.n = pl.words = 0;
+  return pl;
+}
+
+// Bytes of workspace that cover either form of the per-channel quantizer, for every element type.
+int64_t channel_ws_bytes(int64_t BH, int64_t S, int64_t D) {
+  int64_t nsb, rpb;
+  channel_blocking(BH, S, &nsb, &rpb);
+  int64_t b = BH * nsb * D * static_cast<int64_t>(sizeof(float));
+  for (const int e : {2, 4}) {
+    const int64_t w = 4 * once_plan(BH, S, D, e).words;
+    if (w > b) b = w;
+  }
+  return b;
+}
+
 // Lanes per row: the power of two that covers D / 8 lanes (8 channels each);
 // the lanes past D / 8 idle.
 #define FADE_DISPATCH_LPR(D, ...)                                        \
@@ -842,26 +1186,48 @@ void channel_blocking(int64_t BH, int64_t S, int64_t* nsb, int64_t* rows_per_blo
   else if ((D) <= 128) { constexpr int LPR = 16; __VA_ARGS__; }          \
   else { constexpr int LPR = 32; __VA_ARGS__; }
 
+template <typename InT, int MODE, int BITS, int LPR, int NR, bool NT = false>
+void launch_once(const InT* x, int64_t BH, int64_t H, int64_t S, int64_t D, int64_t sb, int64_t sh, int64_t ss,
+                 void* packed, void* scale, uint32_t* ws, const OncePlan& pl, int polls, hipStream_t st) {
+  if (pl.n > 1)
+    hipLaunchKernelGGL(zero_words_kernel, dim3(static_cast<unsigned>(cdiv(pl.words, kBlock))), dim3(kBlock), 0, st, ws, pl.words);
+  hipLaunchKernelGGL((quant_channel_once_kernel<InT, MODE, BITS, LPR, NR, NT>),
+                     dim3(static_cast<unsigned>(pl.n), static_cast<unsigned>(BH)), dim3(kBlock), 0, st, x,
+                     static_cast<int>(D), H, S, sb, sh, ss, ws, polls, static_cast<uint8_t*>(packed),
+                     static_cast<typename ScaleOf<MODE>::T*>(scale));
+}
+
 template <typename InT, int MODE, int BITS>
 int launch_channel(const char* fn, const InT* x, int64_t B, int64_t H, int64_t S, int64_t D,
                    int64_t sb, int64_t sh, int64_t ss, void* packed, void* scale, void* ws,
-                   int64_t ws_bytes, hipStream_t st) {
+                   int64_t ws_bytes, hipStream_t st, int polls = kPolls) {
   const int64_t BH = B * H;
   if (BH == 0) return FADE_OK;
   if (S == 0) return einval("%s: S must be > 0 for a per-channel scale", fn);
-  int64_t nsb, rpb;
-  channel_blocking(BH, S, &nsb, &rpb);
-  const int64_t need = BH * nsb * D * static_cast<int64_t>(sizeof(float));
+  const int64_t need = channel_ws_bytes(BH, S, D);
   if (ws == nullptr || ws_bytes < need)
     return einval("%s: workspace too small (%lld < %lld bytes)", fn, (long long)ws_bytes, (long long)need);
   if (BH > 65535) return einval("%s: B*H=%lld exceeds 65535", fn, (long long)BH);
-  dim3 grid(static_cast<unsigned>(nsb), static_cast<unsigned>(BH));
+  const OncePlan pl = once_plan(BH, S, D, sizeof(InT));
+  constexpr int kBig = sizeof(InT) == 2 ? 16 : 8, kSmall = kBig / 4;
+  uint32_t* area = static_cast<uint32_t*>(ws);
   FADE_DISPATCH_LPR(D, {
-    hipLaunchKernelGGL((colmax_kernel<InT, LPR>), grid, dim3(kBlock), 0, st, x, static_cast<int>(D), H, S, sb, sh, ss,
-                       rpb, static_cast<float*>(ws));
-    hipLaunchKernelGGL((quant_channel_kernel<InT, MODE, BITS, LPR>), grid, dim3(kBlock), 0, st, x,
-                       static_cast<int>(D), H, S, sb, sh, ss, rpb, static_cast<const float*>(ws), static_cast<int>(nsb),
-                       static_cast<uint8_t*>(packed), static_cast<typename ScaleOf<MODE>::T*>(scale));
+    if (sizeof(InT) == 2 && pl.n > 0 && pl.big && BH * S * D * sizeof(InT) >= kStreamBytes) {
+      launch_once<InT, MODE, BITS, LPR, kBig, sizeof(InT) == 2>(x, BH, H, S, D, sb, sh, ss, packed, scale, area, pl, polls, st);
+    } else if (pl.n > 0 && pl.big) {
+      launch_once<InT, MODE, BITS, LPR, kBig>(x, BH, H, S, D, sb, sh, ss, packed, scale, area, pl, polls, st);
+    } else if (pl.n > 0) {
+      launch_once<InT, MODE, BITS, LPR, kSmall>(x, BH, H, S, D, sb, sh, ss, packed, scale, area, pl, polls, st);
+    } else {
+      int64_t nsb, rpb;
+      channel_blocking(BH, S, &nsb, &rpb);
+      dim3 grid(static_cast<unsigned>(nsb), static_cast<unsigned>(BH));
+      hipLaunchKernelGGL((colmax_kernel<InT, LPR>), grid, dim3(kBlock), 0, st, x, static_cast<int>(D), H, S, sb, sh, ss,
+                         rpb, static_cast<float*>(ws));
+      hipLaunchKernelGGL((quant_channel_kernel<InT, MODE, BITS, LPR>), grid, dim3(kBlock), 0, st, x,
+                         static_cast<int>(D), H, S, sb, sh, ss, rpb, static_cast<const float*>(ws), static_cast<int>(nsb),
+                         static_cast<uint8_t*>(packed), static_cast<typename ScaleOf<MODE>::T*>(scale));
+    }
   });
   return check_launch(fn);
 }
@@ -942,9 +1308,7 @@ FADE_API int fade_unpack_codes(const void* packed_u8, int64_t n_rows, int64_t D,
 FADE_API int fade_quant_k_int4_workspace_bytes(int64_t B, int64_t H, int64_t S, int64_t D,
                                                int64_t* bytes) {
   if (bytes == nullptr) return einval("fade_quant_k_int4_workspace_bytes: null output");
-  int64_t nsb, rpb;
-  channel_blocking(B * H, S, &nsb, &rpb);
-  *bytes = B * H * nsb * D * static_cast<int64_t>(sizeof(float));
+  *bytes = channel_ws_bytes(B * H, S, D);
   return FADE_OK;
 }
 
@@ -987,6 +1351,13 @@ FADE_API int fade_quant_v_int4(const void* v_f16, int64_t B, int64_t H, int64_t 
 FADE_API int fade_quant_k_int4_dtype(const void* k, int32_t dtype, int64_t B, int64_t H, int64_t S, int64_t D,
                                      int64_t sb, int64_t sh, int64_t ss, void* packed_u8, void* scale,
                                      void* workspace, int64_t workspace_bytes, void* stream) {
+  return fade_quant_k_int4_polls(k, dtype, B, H, S, D, sb, sh, ss, kPolls, packed_u8, scale, workspace, workspace_bytes,
+                                 stream);
+}
+
+FADE_API int fade_quant_k_int4_polls(const void* k, int32_t dtype, int64_t B, int64_t H, int64_t S, int64_t D,
+                                     int64_t sb, int64_t sh, int64_t ss, int32_t polls, void* packed_u8, void* scale,
+                                     void* workspace, int64_t workspace_bytes, void* stream) {
   const char* fn = "fade_quant_k_int4_dtype";
   int rc = check_dims(fn, B, H, S, D);
   if (rc) return rc;
@@ -995,13 +1366,13 @@ FADE_API int fade_quant_k_int4_dtype(const void* k, int32_t dtype, int64_t B, in
   switch (dtype) {
     case FADE_DTYPE_F16:
       return launch_channel<uint16_t, MODE_F16, 4>(fn, static_cast<const uint16_t*>(k), B, H, S, D, sb, sh, ss,
-                                                   packed_u8, scale, workspace, workspace_bytes, as_stream(stream));
+                                                   packed_u8, scale, workspace, workspace_bytes, as_stream(stream), polls);
     case FADE_DTYPE_BF16:
       return launch_channel<Bf16, MODE_BF16, 4>(fn, static_cast<const Bf16*>(k), B, H, S, D, sb, sh, ss, packed_u8,
-                                                scale, workspace, workspace_bytes, as_stream(stream));
+                                                scale, workspace, workspace_bytes, as_stream(stream), polls);
     case FADE_DTYPE_F32:
       return launch_channel<float, MODE_F32S, 4>(fn, static_cast<const float*>(k), B, H, S, D, sb, sh, ss,
-                                                 packed_u8, scale, workspace, workspace_bytes, as_stream(stream));
+                                                 packed_u8, scale, workspace, workspace_bytes, as_stream(stream), polls);
     default: return einval("%s: unknown dtype %d", fn, dtype);
   }
 }

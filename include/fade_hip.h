@@ -102,6 +102,12 @@ int fade_dequant_sym(const void* packed_u8, const void* scale_f16, int32_t bits,
 int fade_quant_k_int4_dtype(const void* k, int32_t dtype, int64_t B, int64_t H, int64_t S, int64_t D, int64_t sb,
                             int64_t sh, int64_t ss, void* packed_u8, void* scale, void* workspace,
                             int64_t workspace_bytes, void* stream);
+/* The same with the most polls of the wait in which the workgroups of one
+ * (b, h) exchange their column maxima (0 .. INT32_MAX; a workgroup that stops
+ * waiting computes them itself, with the same results). */
+int fade_quant_k_int4_polls(const void* k, int32_t dtype, int64_t B, int64_t H, int64_t S, int64_t D, int64_t sb,
+                            int64_t sh, int64_t ss, int32_t polls, void* packed_u8, void* scale, void* workspace,
+                            int64_t workspace_bytes, void* stream);
 int fade_quant_v_int4_dtype(const void* v, int32_t dtype, int64_t B, int64_t H, int64_t S, int64_t D, int64_t sb,
                             int64_t sh, int64_t ss, void* packed_u8, void* scale, void* stream);
 /* out = dtype(code * scale), scale and out both of `dtype`. */
