@@ -512,29 +512,74 @@ __global__ __launch_bounds__(kThreads) void decode_valu_kernel(Params p) {
 
 }  // namespace
 
-// Merge the n_splits partials of each (b, hq) into the fp16 output; one
-// thread per channel (blockDim.x = head_dim D).
-__global__ __launch_bounds__(256) void decode_combine_kernel(const float* __restrict__ ws_ml,
-                                                             const float* __restrict__ ws_acc,
-                                                             int n_splits, int64_t Hq,
-                                                             uint16_t* __restrict__ out,
-                                                             int64_t o_sb, int64_t o_sh, int bf16) {
+// Merge the n_splits partials of (b, hq) = blockIdx.x into the 16-bit output:
+// D / 4 threads take four channels of a split each, 1024 / D splits at a time,
+// and the slices are summed through LDS in a fixed order.  The first kAhead
+// rounds of partials are loaded before the maximum over the splits is known, so
+// a call of up to 4096 / D splits waits for memory once (one thread per channel
+// walking the splits in turn waited for each: 14 heads x 17 splits at head_dim
+// 64 8.7 -> 3.9 us).
+__global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(const float* __restrict__ ws_ml,
+                                                                         const float* __restrict__ ws_acc, int n_splits,
+                                                                         int64_t Hq, int D, uint16_t* __restrict__ out,
+                                                                         int64_t o_sb, int64_t o_sh, int bf16) {
+  constexpr int kAhead = 4, kW = kCombineThreads / 64;
   const int64_t bh = blockIdx.x;
-  const int d = threadIdx.x, D = blockDim.x;
+  const int tpr = D / 4, slices = kCombineThreads / tpr;
+  const int tid = threadIdx.x, c = tid % tpr, slice = tid / tpr;  // threads past the slices idle
   const float* ml = ws_ml + bh * n_splits * 2;
-  float M = -INFINITY;
-  for (int s = 0; s < n_splits; ++s) M = fmaxf(M, ml[2 * s]);
-  float L = 0.0f, o = 0.0f;
-  if (M != -INFINITY) {
-    for (int s = 0; s < n_splits; ++s) {
-      const float m = ml[2 * s];
-      if (m == -INFINITY) continue;
-      const float w = exp2f(m - M);
-      L += ml[2 * s + 1] * w;
-      o += ws_acc[(bh * n_splits + s) * D + d] * w;
-    }
+  const float* acc = ws_acc + bh * n_splits * D + 4 * c;
+  __shared__ float wmax[kW];
+  __shared__ float4 red[kCombineThreads];
+  __shared__ float red_l[kCombineThreads];
+  auto at = [&](int i) { return slice < slices ? slice + i * slices : n_splits; };
+  float4 a[kAhead];
+  float2 w[kAhead];
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) {
+    const int s = at(i) < n_splits ? at(i) : 0;  // past the splits: loaded, not used
+    a[i] = *reinterpret_cast<const float4*>(acc + static_cast<int64_t>(s) * D);
+    w[i] = *reinterpret_cast<const float2*>(ml + 2 * s);
   }
-  out[(bh / Hq) * o_sb + (bh % Hq) * o_sh + d] = bf16 ? f2bf(o / L) : f2h(o / L);
+  float M = -INFINITY;
+  for (int s = tid; s < n_splits; s += kCombineThreads) M = fmaxf(M, ml[2 * s]);
+  M = group_max<64>(M);
+  if ((tid & 63) == 0) wmax[tid >> 6] = M;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kW; ++k) M = fmaxf(M, wmax[k]);
+  float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float L = 0.0f;
+  auto add = [&](const float4& v, const float2& p) {
+    if (p.x == -INFINITY) return;  // an empty split
+    const float f = exp2f(p.x - M);
+    L += p.y * f;
+    o.x += v.x * f;
+    o.y += v.y * f;
+    o.z += v.z * f;
+    o.w += v.w * f;
+  };
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i)
+    if (at(i) < n_splits) add(a[i], w[i]);
+  for (int i = kAhead; at(i) < n_splits; ++i)
+    add(*reinterpret_cast<const float4*>(acc + static_cast<int64_t>(at(i)) * D), *reinterpret_cast<const float2*>(ml + 2 * at(i)));
+  red[tid] = o;
+  red_l[tid] = L;
+  __syncthreads();
+  if (tid >= tpr) return;
+  for (int k = 1; k < slices; ++k) {
+    const float4 v = red[k * tpr + c];
+    o.x += v.x;
+    o.y += v.y;
+    o.z += v.z;
+    o.w += v.w;
+    L += red_l[k * tpr + c];
+  }
+  const float y[4] = {o.x / L, o.y / L, o.z / L, o.w / L};
+  uint16_t* dst = out + (bh / Hq) * o_sb + (bh % Hq) * o_sh + 4 * c;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) dst[k] = bf16 ? f2bf(y[k]) : f2h(y[k]);
 }
 
 int launch_valu(const Params& p, hipStream_t st) {

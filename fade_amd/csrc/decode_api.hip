@@ -286,8 +286,8 @@ int run_plan(const fade_decode_args* a, Params& p, const Plan& pl, uint32_t* cou
   if (rc) return rc;
   if (pl.k == Kern::kValu && p.n_splits == 1) return 0;  // the portable kernel wrote the output
   const int64_t rows = a->B * a->Hq;
-  hipLaunchKernelGGL(decode_combine_kernel, dim3(static_cast<unsigned>(rows)), dim3(static_cast<unsigned>(p.D)), 0, st, p.ws_ml,
-                     p.ws_acc, p.n_splits, a->Hq, static_cast<uint16_t*>(a->out), a->o_sb, a->o_sh, p.bf16);
+  hipLaunchKernelGGL(decode_combine_kernel, dim3(static_cast<unsigned>(rows)), dim3(kCombineThreads), 0, st, p.ws_ml,
+                     p.ws_acc, p.n_splits, a->Hq, p.D, static_cast<uint16_t*>(a->out), a->o_sb, a->o_sh, p.bf16);
   return check_launch("fade_tiered_decode_attn(combine)");
 }
 

@@ -96,9 +96,9 @@ __device__ __forceinline__ int asym_code_at(const uint8_t* row, int d, int bits)
   return (byte >> (6 - 2 * (d & 3))) & 3;
 }
 
-__global__ void decode_combine_kernel(const float* __restrict__ ws_ml,
-                                      const float* __restrict__ ws_acc, int n_splits, int64_t Hq,
-                                      uint16_t* __restrict__ out, int64_t o_sb, int64_t o_sh, int bf16);
+constexpr int kCombineThreads = 256;
+__global__ void decode_combine_kernel(const float* __restrict__ ws_ml, const float* __restrict__ ws_acc, int n_splits,
+                                      int64_t Hq, int D, uint16_t* __restrict__ out, int64_t o_sb, int64_t o_sh, int bf16);
 
 int launch_valu(const Params& p, hipStream_t st);
 // Matrix-core kernel; returns FADE_EINVAL when the middle format is not handled.
