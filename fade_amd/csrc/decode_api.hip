@@ -204,15 +204,47 @@ struct Plan {
   int64_t n, tps, n_f16_tiles, tiles_per_split;
 };
 
+// Splits of `tiles` tiles for the packed kernel, `pairs` workgroups per split: at
+// most the count that fills the resident workgroup slots (large caches take
+// it), fewer where the merge costs more than the added workgroups gain.
+// Estimated time in us, from sweeps of forced split counts over B = 1 .. 16 and
+// 600 .. 32K tokens in every format: a wave walks its tiles one at a time, kTile
+// us each (more where two workgroups share a CU, which hides little latency a
+// lone one does not), a further round of workgroups starts over, and a merge
+// costs a round trip through memory plus its splits.  Measured, one-wave rule ->
+// this: B=1, 32/8 heads, 2048 tokens 18.1 -> 9.9 us (34 one-tile splits -> 9),
+// 16K tokens 24.4 -> 16.6 (64 -> 22), B=4 at 4096 15.4 -> 13.2, B=8, 28/4 heads at
+// 470 tokens 11.3 -> 9.7; B=16 at 8192 and the 32K formats as before.
+int64_t packed_splits(int64_t pairs, int64_t tiles, int waves, int resident) {
+  const int64_t cus = num_cus(), per_cu = resident / cus > 0 ? resident / cus : 1;
+  const double kTile = waves == 4 ? 1.55 : 2.0, kShared = 0.5, kStart = 3.0, kMerge = 1.0, kSplit = 0.25;
+  int64_t most = (resident + pairs / 2) / pairs;
+  if (most > tiles) most = tiles;
+  int64_t best = 1;
+  double best_us = 0.0;
+  for (int64_t want = 1; want <= most; ++want) {
+    const int64_t per = cdiv(tiles, want), n = cdiv(tiles, per), on_cu = cdiv(pairs * n, cus);
+    const int64_t rounds = on_cu / per_cu, rest = on_cu % per_cu;
+    // tiles of a wave: the waves claim them one at a time, so between the mean and its ceiling
+    const double walk = 0.5 * (static_cast<double>(cdiv(per, waves)) + static_cast<double>(per) / waves);
+    auto round_us = [&](int64_t g) { return kStart + walk * kTile * (1.0 + kShared * (g - 1)); };
+    const double us = rounds * round_us(per_cu) + (rest > 0 ? round_us(rest) : 0.0) + (n > 1 ? kMerge + kSplit * n : 0.0);
+    if (want == 1 || us < best_us) {
+      best = n;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 Plan make_plan(const fade_decode_args* a, const Params& p) {
   Plan pl{};
   pl.k = choose(a, p);
   if (pl.k == Kern::kInt4) {
-    // One machine-wide wave of resident workgroups; tiles of either kind cost
-    // about the same bytes (8 KB), so splits take equal tile counts.
+    // tiles of either kind cost about the same bytes (8 KB), so splits take equal tile counts
     const int64_t nT = int4_tiles(p);
     const int64_t pairs = a->B * a->Hkv * int4_grid_passes(p);  // workgroups per split
-    int64_t want = a->n_splits > 0 ? a->n_splits : (int4_resident_wgs(p) + pairs / 2) / pairs;
+    int64_t want = a->n_splits > 0 ? a->n_splits : packed_splits(pairs, nT, int4_waves(p), int4_resident_wgs(p));
     pl.n_f16_tiles = int4_fp16_tiles(p);
     pl.tps = 0;
     if (p.rot != nullptr) {

@@ -112,6 +112,7 @@ int int4_fp16_tiles(const Params& p);
 int64_t int4_tiles(const Params& p);
 int int4_resident_wgs(const Params& p);  // resident workgroups of the kernel instance for p
 int int4_grid_passes(const Params& p);   // head passes the instance's grid carries per kv head
+int int4_waves(const Params& p);         // wavefronts of the instance's workgroups
 bool eight_heads_pay(const Params& p);   // GQA 5..8, symmetric tier: one eight-head pass rather than two
 int launch_int4(const Params& p, hipStream_t st);
 // A packed-kernel instance: the kernel, its wavefronts per workgroup, and its

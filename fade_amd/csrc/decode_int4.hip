@@ -146,6 +146,7 @@ int int4_resident_wgs(const Params& p) {
 }
 
 int int4_grid_passes(const Params& p) { return packed_kernel(p).grid_passes; }
+int int4_waves(const Params& p) { return packed_kernel(p).waves; }
 
 int launch_int4(const Params& p, hipStream_t st) {
   const Choice c = packed_kernel(p);
