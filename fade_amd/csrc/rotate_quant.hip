@@ -35,6 +35,12 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kD = 128;
 constexpr int kWaves = 8;
 constexpr int kThreads = 64 * kWaves;
+// Waves of the per-token kernel: four per SIMD, no tile loaded ahead (config 2's
+// 1.04 M rows: 81 us; two per SIMD with the next tile in flight 87).  The
+// per-channel passes keep 8 waves with two tiles each per R fragment (163 us for
+// both; 16 waves of one tile: 173).
+constexpr int kTokenWaves = 16;
+constexpr int kTokenThreads = 64 * kTokenWaves;
 constexpr int kRows = 32;     // rows per wave tile
 constexpr int kRPitch = 136;  // halves per R row in LDS: 16-byte reads of 8 rows hit distinct banks
 constexpr float kRScale = 1024.0f;         // R is carried as 2^10 R
@@ -76,20 +82,27 @@ __device__ __forceinline__ int64_t row_off(const Geom& gm, int64_t r) {
   return gm.fs ? r * gm.fs : row_offset(r, gm.H, gm.S, gm.sb, gm.sh, gm.ss);
 }
 
-// R (fp32 [128][128], row-major, 16-byte aligned) -> R_hi / R_lo rows in LDS.
+// R (fp32 [128][128], row-major, 16-byte aligned) -> R_hi / R_lo rows in LDS, four
+// channels (8 bytes) per write: a wave writes two rows at a time, 32 lanes over
+// a row's 64 banks.
+template <int THREADS>
 __device__ __forceinline__ void load_r(const float* __restrict__ R, RTile& rt) {
-  for (int e = threadIdx.x; e < kD * kD / 4; e += kThreads) {
+#pragma unroll
+  for (int k = 0; k < kD * kD / 4 / THREADS; ++k) {
+    const int e = threadIdx.x + k * THREADS;
     const float4 v = reinterpret_cast<const float4*>(R)[e];
     const int row = e >> 5, col = (e & 31) * 4;
     const float f[4] = {v.x, v.y, v.z, v.w};
+    uint32_t h[4], l[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float fs = f[j] * kRScale;  // exact
-      const _Float16 h = static_cast<_Float16>(fs);
-      const _Float16 l = static_cast<_Float16>(fs - static_cast<float>(h));
-      rt.hi[row][col + j] = __builtin_bit_cast(uint16_t, h);
-      rt.lo[row][col + j] = __builtin_bit_cast(uint16_t, l);
+      const _Float16 hj = static_cast<_Float16>(fs);
+      h[j] = __builtin_bit_cast(uint16_t, hj);
+      l[j] = __builtin_bit_cast(uint16_t, static_cast<_Float16>(fs - static_cast<float>(hj)));
     }
+    *reinterpret_cast<uint2*>(&rt.hi[row][col]) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
+    *reinterpret_cast<uint2*>(&rt.lo[row][col]) = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
   }
 }
 
@@ -218,30 +231,26 @@ __device__ __forceinline__ void flush_stage(const uint8_t* stage, uint8_t* __res
 }
 
 // Per-token scales: the waves of the grid take 32-row tiles of the flattened
-// [B*H*S] rows in turn; the next tile's x is in flight during this one.
+// [B*H*S] rows in turn.  Bound by the matrix cores and the issue around them:
+// without the loads of x it takes 70 us, with half the MFMAs 69.
 template <int BITS>
-__global__ __launch_bounds__(kThreads) void rotq_token_kernel(const uint16_t* __restrict__ x, Geom gm, int64_t rows,
+__global__ __launch_bounds__(kTokenThreads) void rotq_token_kernel(const uint16_t* __restrict__ x, Geom gm, int64_t rows,
                                                               const float* __restrict__ R,
                                                               uint8_t* __restrict__ packed,
                                                               uint16_t* __restrict__ scale) {
   constexpr float QMAX = static_cast<float>(RQ<BITS>::hi);
   __shared__ __attribute__((aligned(16))) RTile rt;
-  __shared__ __attribute__((aligned(16))) uint8_t stage[kWaves][kRows * StagePitch<BITS>::value];
-  load_r(R, rt);
+  __shared__ __attribute__((aligned(16))) uint8_t stage[kTokenWaves][kRows * StagePitch<BITS>::value];
+  load_r<kTokenThreads>(R, rt);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
-  const int64_t step = static_cast<int64_t>(gridDim.x) * kWaves * kRows;
-  int64_t r0 = (static_cast<int64_t>(blockIdx.x) * kWaves + wave) * kRows;
+  const int64_t step = static_cast<int64_t>(gridDim.x) * kTokenWaves * kRows;
+  int64_t r0 = (static_cast<int64_t>(blockIdx.x) * kTokenWaves + wave) * kRows;
   const int64_t last = rows - 1;
-  f16x8 xb[8];
-  load_x(x, row_off(gm, r0 + n < rows ? r0 + n : last), h, xb);
   for (; r0 < rows; r0 += step) {
     __asm__ volatile("" ::: "memory");  // keep the R fragment reads inside the loop
     f16x8 cur[8];
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) cur[ks] = xb[ks];
-    const int64_t nx = r0 + step + n;
-    load_x(x, row_off(gm, nx < rows ? nx : last), h, xb);
+    load_x(x, row_off(gm, r0 + n < rows ? r0 + n : last), h, cur);
     f32x16 xr[4];
     float a = 0.0f;
 #pragma unroll
@@ -266,7 +275,7 @@ __global__ __launch_bounds__(kThreads) void rotq_colmax_kernel(const uint16_t* _
                                                                float* __restrict__ partial) {
   __shared__ __attribute__((aligned(16))) RTile rt;
   __shared__ float red[kWaves][kD];
-  load_r(R, rt);
+  load_r<kThreads>(R, rt);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
   const int64_t bh = blockIdx.y;
@@ -329,7 +338,7 @@ __global__ __launch_bounds__(kThreads) void rotq_channel_kernel(const uint16_t* 
   __shared__ __attribute__((aligned(16))) RTile rt;
   __shared__ __attribute__((aligned(16))) uint8_t stage[kWaves][2 * kRows * StagePitch<BITS>::value];
   __shared__ float inv_s[kD];
-  load_r(R, rt);
+  load_r<kThreads>(R, rt);
   const int64_t bh = blockIdx.y;
   const int nsb = gridDim.x;
   for (int d = threadIdx.x; d < kD; d += kThreads) {
@@ -439,13 +448,13 @@ FADE_API int fade_rotate_quant(const void* x_f16, int64_t B, int64_t H, int64_t 
   uint16_t* sc = static_cast<uint16_t*>(scale_f16);
   hipStream_t st = as_stream(stream);
   if (axis == FADE_AXIS_TOKEN) {
-    const int64_t want = cdiv(rows, static_cast<int64_t>(kRows) * kWaves);
+    const int64_t want = cdiv(rows, static_cast<int64_t>(kRows) * kTokenWaves);
     const int64_t cap = num_cus();
     const dim3 grid(static_cast<unsigned>(want < cap ? want : cap));
     switch (bits) {
-      case 4: hipLaunchKernelGGL(rotq_token_kernel<4>, grid, dim3(kThreads), 0, st, x, gm, rows, R, pk, sc); break;
-      case 3: hipLaunchKernelGGL(rotq_token_kernel<3>, grid, dim3(kThreads), 0, st, x, gm, rows, R, pk, sc); break;
-      default: hipLaunchKernelGGL(rotq_token_kernel<2>, grid, dim3(kThreads), 0, st, x, gm, rows, R, pk, sc); break;
+      case 4: hipLaunchKernelGGL(rotq_token_kernel<4>, grid, dim3(kTokenThreads), 0, st, x, gm, rows, R, pk, sc); break;
+      case 3: hipLaunchKernelGGL(rotq_token_kernel<3>, grid, dim3(kTokenThreads), 0, st, x, gm, rows, R, pk, sc); break;
+      default: hipLaunchKernelGGL(rotq_token_kernel<2>, grid, dim3(kTokenThreads), 0, st, x, gm, rows, R, pk, sc); break;
     }
     return check_launch(fn);
   }
