@@ -192,6 +192,9 @@ _SIGNATURES: dict[str, list] = {
     "fade_tiered_decode_workspace_bytes": [ctypes.POINTER(DecodeArgs), _pi64],
     "fade_tiered_decode_attn": [ctypes.POINTER(DecodeArgs), _p],
     "fade_tiered_decode_attn_noalloc": [ctypes.POINTER(DecodeArgs), _p],
+    "fade_append_rows": [
+        _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i64, _p,
+    ],
     "fade_reassign_plan": [_p, _i64, _i64, _i64, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _p],
     "fade_reassign_gather": [ctypes.POINTER(ReassignArgs), _p],
     "fade_tiered_prefill_attn": [ctypes.POINTER(PrefillArgs), _p],
@@ -284,6 +287,20 @@ def require_gpu(*tensors: torch.Tensor | None, op: str = "fade_amd") -> None:
             dev = t.device
         elif t.device != dev:
             raise ValueError(f"{op}: tensors are on different devices ({dev} vs {t.device})")
+
+
+def plain(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel may stand in for tensor ops on these: plain tensors that record no
+    gradient, outside forward-mode, functorch transforms and compilation."""
+    if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
+            return False
+        if (grad and t.requires_grad) or torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return False
+    return True
 
 
 # FADE_DTYPE_* of the dtype-tagged quantizer entry points

@@ -136,6 +136,32 @@ def _sel(x: Tensor, idx: Tensor) -> Tensor:
     return x.index_select(-2, idx).contiguous()
 
 
+def _append_rows(k: Tensor, v: Tensor, bk: Tensor, bv: Tensor, bp: Tensor, at: int, pos0: int) -> bool:
+    """Rows ``k``, ``v`` into the buffers from row ``at`` on and their positions, in one
+    launch (``fade_append_rows``).  False, with nothing done, for what that kernel does not
+    copy as it is: other devices or dtypes than the buffers', rows that are not whole 16-byte
+    units, tensors that record gradients, subclasses and tracing."""
+    if not (k.is_cuda and k.device == v.device == bk.device and _lib.plain(k, v, bk, bv)):
+        return False
+    es = k.element_size()
+    if k.dtype != bk.dtype or v.dtype != bv.dtype or k.dtype != v.dtype or es not in (2, 4):
+        return False
+    B, H, n, D = k.shape
+    if v.shape != k.shape or bk.shape[0] != B or bk.shape[1] != H or bk.shape[3] != D or bv.shape != bk.shape:
+        return False
+    if B * H > 65535 or n * D * es >= 1 << 35:
+        return False
+    ks, vs, per = k.stride(), v.stride(), 16 // es
+    if ks[3] != 1 or vs[3] != 1 or (D | ks[0] | ks[1] | ks[2] | vs[0] | vs[1] | vs[2]) % per:
+        return False
+    kp, vp = k.data_ptr(), v.data_ptr()
+    if (kp | vp | bk.data_ptr() | bv.data_ptr()) % 16 or not (bk.is_contiguous() and bv.is_contiguous()):
+        return False
+    _lib.call("fade_append_rows", kp, ks[0], ks[1], ks[2], vp, vs[0], vs[1], vs[2], es, B, H, n, D, bk.data_ptr(),
+              bv.data_ptr(), bp.data_ptr(), bk.shape[2], at, pos0, _lib.current_stream_handle(k.device))
+    return True
+
+
 class TieredKVCache(DynamicCache):
     """Tiered KV cache with attention-aware compression (fade/cache.py:136-225).
 
@@ -459,29 +485,24 @@ class TieredKVCache(DynamicCache):
             self._append_fp16_ragged(st, k, v)
             return
         n = int(k.shape[-2])
-        new_pos = torch.arange(st.next_position, st.next_position + n, device=k.device)
+        pos0 = st.next_position
         st.next_position += n
         if st._fp16_buf_k is None:
-            have = 0 if st.fp16_k is None else int(st.fp16_k.shape[-2])
-            need = have + n
-            cap = max(DEFAULT_FP16_PREALLOC, need)
+            old = 0 if st.fp16_k is None else int(st.fp16_k.shape[-2])
+            cap = max(DEFAULT_FP16_PREALLOC, old + n)
             B, H, _, D = k.shape
             st._fp16_buf_k = torch.empty(B, H, cap, D, dtype=k.dtype, device=k.device)
             st._fp16_buf_v = torch.empty(B, H, cap, D, dtype=v.dtype, device=v.device)
             st._fp16_buf_pos = torch.empty(cap, dtype=torch.long, device=k.device)
-            if have:
-                st._fp16_buf_k[:, :, :have] = st.fp16_k
-                st._fp16_buf_v[:, :, :have] = st.fp16_v
-                st._fp16_buf_pos[:have] = st.fp16_pos
-            st._fp16_buf_k[:, :, have:need] = k
-            st._fp16_buf_v[:, :, have:need] = v
-            st._fp16_buf_pos[have:need] = new_pos
-            st._fp16_len = need
+            if old:
+                st._fp16_buf_k[:, :, :old] = st.fp16_k
+                st._fp16_buf_v[:, :, :old] = st.fp16_v
+                st._fp16_buf_pos[:old] = st.fp16_pos
         else:
-            old, new = st._fp16_len, st._fp16_len + n
+            old = st._fp16_len
             cap = st._fp16_buf_k.shape[-2]
-            if new > cap:
-                cap2 = max(cap * 2, new)
+            if old + n > cap:
+                cap2 = max(cap * 2, old + n)
                 B, H, _, D = st._fp16_buf_k.shape
                 bk = torch.empty(B, H, cap2, D, dtype=k.dtype, device=k.device)
                 bv = torch.empty(B, H, cap2, D, dtype=v.dtype, device=v.device)
@@ -490,10 +511,11 @@ class TieredKVCache(DynamicCache):
                 bv[:, :, :old] = st._fp16_buf_v[:, :, :old]
                 bp[:old] = st._fp16_buf_pos[:old]
                 st._fp16_buf_k, st._fp16_buf_v, st._fp16_buf_pos = bk, bv, bp
-            st._fp16_buf_k[:, :, old:new] = k
-            st._fp16_buf_v[:, :, old:new] = v
-            st._fp16_buf_pos[old:new] = new_pos
-            st._fp16_len = new
+        if not _append_rows(k, v, st._fp16_buf_k, st._fp16_buf_v, st._fp16_buf_pos, old, pos0):
+            st._fp16_buf_k[:, :, old : old + n] = k
+            st._fp16_buf_v[:, :, old : old + n] = v
+            st._fp16_buf_pos[old : old + n] = torch.arange(pos0, pos0 + n, device=k.device)
+        st._fp16_len = old + n
         ln = st._fp16_len
         st.fp16_k = st._fp16_buf_k[:, :, :ln]
         st.fp16_v = st._fp16_buf_v[:, :, :ln]

@@ -275,10 +275,67 @@ __global__ __launch_bounds__(256) void gather_kernel(FadeReassignArgs a) {
   }
 }
 
+// Appends n rows per (b, h) = blockIdx.y to the fp16 tier's K and V buffers
+// ([B,H,cap,*] contiguous, from row `at` on) and their positions, in 16-byte
+// units of either tensor.  A decode step appends one row: the launch is all it
+// costs, where the tensor ops it replaces (three copies, an arange) were 30 us of
+// host time per layer and token; a prompt moves at the copy rate.
+struct AppendArgs {
+  const uint4* k;
+  const uint4* v;
+  int64_t ksb, ksh, kss, vsb, vsh, vss;  // strides in 16-byte units
+  uint4* buf_k;
+  uint4* buf_v;
+  int64_t* buf_pos;
+  int64_t H, cap, at, pos0;
+  uint32_t n, row;  // rows; units of a row
+};
+__global__ __launch_bounds__(256) void append_kernel(AppendArgs a) {
+  const uint32_t bh = blockIdx.y, units = a.n * a.row;
+  const int64_t b = bh / static_cast<uint32_t>(a.H), h = bh % static_cast<uint32_t>(a.H);
+  const uint4* k = a.k + b * a.ksb + h * a.ksh;
+  const uint4* v = a.v + b * a.vsb + h * a.vsh;
+  const int64_t out = (bh * a.cap + a.at) * a.row;
+  for (uint32_t u = blockIdx.x * 256 + threadIdx.x; u < units; u += gridDim.x * 256) {
+    const uint32_t s = u / a.row, c = u - s * a.row;
+    const uint4 x = k[s * a.kss + c], y = v[s * a.vss + c];
+    a.buf_k[out + u] = x;
+    a.buf_v[out + u] = y;
+  }
+  if (bh == 0)
+    for (uint32_t s = blockIdx.x * 256 + threadIdx.x; s < a.n; s += gridDim.x * 256) a.buf_pos[a.at + s] = a.pos0 + s;
+}
+
 }  // namespace
 }  // namespace fade
 
 using namespace fade;
+
+FADE_API int fade_append_rows(const void* k, int64_t ksb, int64_t ksh, int64_t kss, const void* v, int64_t vsb,
+                              int64_t vsh, int64_t vss, int64_t elem_bytes, int64_t B, int64_t H, int64_t n, int64_t D,
+                              void* buf_k, void* buf_v, int64_t* buf_pos, int64_t cap, int64_t at, int64_t pos0,
+                              void* stream) {
+  const char* fn = "fade_append_rows";
+  if (B < 0 || H < 0 || n < 0 || D < 0 || cap < 0 || at < 0) return einval("%s: negative size", fn);
+  if (elem_bytes != 2 && elem_bytes != 4) return einval("%s: elements of 2 or 4 bytes, got %lld", fn, (long long)elem_bytes);
+  if (at > cap || n > cap - at) return einval("%s: rows %lld..%lld of a buffer of %lld", fn, (long long)at, (long long)(at + n), (long long)cap);
+  if (B * H > 65535) return einval("%s: B*H must be at most 65535", fn);
+  if (B * H * n * D == 0) return FADE_OK;
+  if (!k || !v || !buf_k || !buf_v || !buf_pos) return einval("%s: null pointer", fn);
+  const int64_t per = 16 / elem_bytes;  // elements of a unit
+  if ((reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(buf_k) |
+       reinterpret_cast<uintptr_t>(buf_v)) & 15 ||
+      (reinterpret_cast<uintptr_t>(buf_pos) & 7) || (D | ksb | ksh | kss | vsb | vsh | vss) % per)
+    return einval("%s: rows must be whole 16-byte units", fn);
+  if (n * (D / per) >= (int64_t{1} << 31)) return einval("%s: too many rows", fn);
+  const AppendArgs a{static_cast<const uint4*>(k), static_cast<const uint4*>(v), ksb / per, ksh / per, kss / per,
+                     vsb / per, vsh / per, vss / per, static_cast<uint4*>(buf_k), static_cast<uint4*>(buf_v), buf_pos,
+                     H, cap, at, pos0, static_cast<uint32_t>(n), static_cast<uint32_t>(D / per)};
+  const int64_t blocks = cdiv(n * (D / per), 256);
+  hipLaunchKernelGGL(append_kernel, dim3(static_cast<unsigned>(blocks < 1024 ? blocks : 1024), static_cast<unsigned>(B * H)),
+                     dim3(256), 0, as_stream(stream), a);
+  return check_launch(fn);
+}
 
 FADE_API int fade_reassign_plan(const int64_t* tiers, int64_t tiers_row_stride, int64_t rows, int64_t S,
                                 int64_t n_sink, const int64_t* pos_old, int64_t pos_old_row_stride, int32_t* dst,

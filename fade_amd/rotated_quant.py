@@ -155,7 +155,7 @@ def rotated_dequant_rot(packed: Tensor, scale: Tensor, bits: int, dtype: torch.d
 
 def _dequant_fused_ok(packed: Tensor, R: Tensor, bits: int, dtype) -> bool:
     """Whether ``fade_rotate_dequant`` takes this call: its output types and head_dim, rows it
-    can read 16 bytes at a time, and no gradient wanted of R (the kernel records none)."""
+    can read 16 bytes at a time, and plain tensors (the kernel records no gradient of R)."""
     return (
         dtype in (torch.float16, torch.bfloat16)
         and bits in _BIT_PARAMS
@@ -163,7 +163,7 @@ def _dequant_fused_ok(packed: Tensor, R: Tensor, bits: int, dtype) -> bool:
         and packed.is_cuda
         and packed.shape[-1] == (128 if bits == 3 else 16 * bits)
         and tuple(R.shape) == (128, 128)
-        and not (R.requires_grad and torch.is_grad_enabled())
+        and _lib.plain(packed, R)
     )
 
 

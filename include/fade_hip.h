@@ -202,6 +202,15 @@ int fade_rerope_gather_dtype(const void* k, int64_t ksb, int64_t ksh, int64_t ks
                              const float* cos_new, const float* sin_new, void* k_out, void* v_out, int32_t dtype,
                              void* stream);
 
+/* Append n rows to the full-precision tier's buffers (fade/cache.py:608-670):
+ * k, v [B,H,n,D] (element strides, contiguous rows) to rows at .. at + n - 1 of
+ * buf_k, buf_v [B,H,cap,D] contiguous, positions pos0 .. pos0 + n - 1 to
+ * buf_pos[at ..].  Elements of 2 or 4 bytes; rows are whole 16-byte units
+ * (pointers 16-byte aligned, D and strides multiples of 16 / elem_bytes). */
+int fade_append_rows(const void* k, int64_t ksb, int64_t ksh, int64_t kss, const void* v, int64_t vsb, int64_t vsh,
+                     int64_t vss, int64_t elem_bytes, int64_t B, int64_t H, int64_t n, int64_t D, void* buf_k,
+                     void* buf_v, int64_t* buf_pos, int64_t cap, int64_t at, int64_t pos0, void* stream);
+
 /* ---------------- device-side tier reassignment --------------------------- */
 /* fade/cache.py:881-1057 (apply_tier_assignment, shared tiers) for the
  * reference INT4 middle tier, without materializing the layer.

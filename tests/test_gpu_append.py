@@ -1,0 +1,68 @@
+"""``TieredKVCache.update``'s append in one launch (``fade_append_rows``) against tensor copies."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from fade_amd import cache as fc
+
+pytestmark = pytest.mark.gpu
+
+
+def _buffers(B, H, cap, D, dtype, dev):
+    z = lambda *s, **k: torch.full(s, -1, device=dev, **k)  # noqa: E731
+    return z(B, H, cap, D, dtype=dtype), z(B, H, cap, D, dtype=dtype), z(cap, dtype=torch.long)
+
+
+# one row; rows past a block's 256 units; 16-byte rows; a head_dim that is no power of two
+@pytest.mark.parametrize("B,H,n,D,at,cap", [(2, 4, 1, 128, 127, 128), (1, 2, 300, 128, 3, 400), (3, 1, 5, 8, 0, 5), (2, 3, 17, 80, 9, 64),
+                                            (1, 1, 2100, 256, 1, 2101)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_append_rows(dev, B, H, n, D, at, cap, dtype):
+    g = torch.Generator().manual_seed(n)
+    k = torch.randn(B, n, H, D, generator=g).to(dtype).to(dev).transpose(1, 2)  # as a projection's heads come
+    v = torch.randn(B, H, n + 2, D, generator=g).to(dtype).to(dev)[:, :, 2:]
+    bk, bv, bp = _buffers(B, H, cap, D, dtype, dev)
+    want = [t.clone() for t in (bk, bv, bp)]
+    want[0][:, :, at : at + n], want[1][:, :, at : at + n] = k, v
+    want[2][at : at + n] = torch.arange(70, 70 + n, device=dev)
+    assert fc._append_rows(k, v, bk, bv, bp, at, 70)
+    assert all(torch.equal(a, b) for a, b in zip((bk, bv, bp), want))
+
+
+def test_append_rows_left_to_tensor_ops(dev):
+    """Calls the kernel does not take, and the cache's result for them."""
+    r = lambda *s, dt=torch.float16: torch.randn(*s, device=dev).to(dt)  # noqa: E731
+    cases = {
+        "unaligned": (r(1, 2, 3, 129)[..., 1:], r(1, 2, 3, 128)),
+        "short rows": (r(1, 2, 3, 12), r(1, 2, 3, 12)),
+        "strided rows": (r(1, 2, 128, 3).transpose(2, 3), r(1, 2, 3, 128)),
+        "double": (r(1, 2, 3, 128, dt=torch.float64), r(1, 2, 3, 128, dt=torch.float64)),
+        "mixed": (r(1, 2, 3, 128), r(1, 2, 3, 128, dt=torch.float32)),
+        "gradient": (r(1, 2, 3, 128).requires_grad_(), r(1, 2, 3, 128)),
+    }
+    for name, (k, v) in cases.items():
+        bk = torch.zeros(1, 2, 8, k.shape[-1], dtype=k.dtype, device=dev)
+        assert not fc._append_rows(k, v, bk, torch.zeros_like(bk), torch.zeros(8, dtype=torch.long, device=dev), 0, 0), name
+        if name in ("double", "mixed"):
+            continue
+        c = fc.TieredKVCache(n_sink=2, recent_window=4, head_dim=int(k.shape[-1]))
+        c.update(k, v, 0)
+        ko, vo = c.update(k, v, 0)
+        assert torch.equal(ko, torch.cat([k, k], -2)) and torch.equal(vo, torch.cat([v, v], -2)), name
+        assert c._layers[0].fp16_pos.tolist() == list(range(6))
+    k, v = cases["gradient"]
+    c = fc.TieredKVCache(n_sink=2, recent_window=4, head_dim=128)
+    c.update(k, v, 0)[0].float().sum().backward()
+    assert torch.equal(k.grad, torch.ones_like(k))
+
+
+def test_append_grows_and_counts_positions(dev):
+    c = fc.TieredKVCache(n_sink=2, recent_window=4, head_dim=64)
+    parts = [torch.randn(2, 3, n, 64, device=dev).half() for n in (100, 27, 1, 1, 200, 0, 1)]
+    for t in parts:
+        ko, vo = c.update(t, -t, 0)
+    full = torch.cat(parts, -2)
+    assert torch.equal(ko, full) and torch.equal(vo, -full)
+    assert c._layers[0].fp16_pos.tolist() == list(range(330))
