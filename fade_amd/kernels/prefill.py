@@ -125,11 +125,14 @@ class TieredPrefillPlan:
         nb = ctypes.c_int64(0)
         lib.fade_tiered_prefill_workspace_bytes(self._argp, nb)  # (arguments it refuses are refused by run())
         self.workspace = _lib.scratch(nb.value, q.device) if nb.value else None
+        self._ws_stream = _lib.current_stream_handle(q.device) if nb.value else 0
         self._fn = lib.fade_tiered_prefill_attn_ws
 
     def run(self, stream: int | None = None) -> Tensor:
         s = torch.cuda.current_stream(self.out.device).cuda_stream if stream is None else stream
         ws = self.workspace
+        if ws is not None and s != self._ws_stream:  # not reused before that stream is done with it
+            ws.record_stream(torch.cuda.ExternalStream(s, device=self.out.device))
         _lib.check(self._fn(self._argp, None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), s),
                    "fade_tiered_prefill_attn")
         return self.out

@@ -95,3 +95,35 @@ def test_prefill_split_workspace_checked(dev):
     need = plan.workspace.numel()
     assert lib.fade_tiered_prefill_attn_ws(ctypes.byref(plan.args), None, 0, s) == _lib.FADE_EINVAL
     assert lib.fade_tiered_prefill_attn_ws(ctypes.byref(plan.args), plan.workspace.data_ptr(), need - 1, s) == _lib.FADE_EINVAL
+
+
+def test_prefill_split_on_another_stream(dev):
+    """Plans made on one stream, run on another and dropped at once: their sums are not overwritten."""
+    plan = _plan(dev, 1, 4, 1, 128, 16, [(4, 1000, 64)], torch.float16, "bottom_right")
+    want = plan.run().clone()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    outs = []
+    for _ in range(20):
+        p = TieredPrefillPlan(*plan._keep[:5], lens=plan._keep[5])
+        outs.append(p.run(side.cuda_stream))
+        del p
+        torch.full((1 << 20,), 255, dtype=torch.uint8, device=dev)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want) for o in outs)
+
+
+def test_prefill_split_captured(dev):
+    """A captured split call replays to the eager result."""
+    plan = _plan(dev, 1, 14, 2, 64, 70, [(4, 2000, 61)], torch.float16, "bottom_right")
+    want = plan.run().clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plan.run()
+    for _ in range(3):
+        plan.out.zero_()
+        plan.workspace.fill_(255)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(plan.out, want)
