@@ -222,7 +222,7 @@ int64_t packed_splits(int64_t pairs, int64_t tiles, int waves, int resident) {
   if (most > tiles) most = tiles;
   int64_t best = 1;
   double best_us = 0.0;
-  for (int64_t want = 1; want <= most; ++want) {
+  for (int64_t want = 1; want <= most;) {
     const int64_t per = cdiv(tiles, want), n = cdiv(tiles, per), on_cu = cdiv(pairs * n, cus);
     const int64_t rounds = on_cu / per_cu, rest = on_cu % per_cu;
     // tiles of a wave: the waves claim them one at a time, so between the mean and its ceiling
@@ -233,6 +233,8 @@ int64_t packed_splits(int64_t pairs, int64_t tiles, int waves, int resident) {
       best = n;
       best_us = us;
     }
+    if (per == 1) break;
+    want = cdiv(tiles, per - 1);  // the next count that leaves fewer tiles to a split
   }
   return best;
 }

@@ -362,7 +362,7 @@ FADE_API int fade_rotate_dequant(const void* packed, const void* scale, int32_t 
   if (dtype != FADE_DTYPE_F16 && dtype != FADE_DTYPE_BF16)
     return einval("%s: dtype must be FADE_DTYPE_F16 or FADE_DTYPE_BF16, got %d", fn, dtype);
   if (B * H * S == 0) return FADE_OK;
-  if (B * H * S > (int64_t{1} << 38)) return einval("%s: shape too large", fn);  // work items are 32-bit
+  if (B * H * S > (int64_t{1} << 35)) return einval("%s: shape too large", fn);  // work items are 32-bit
   if (packed == nullptr || scale == nullptr || R == nullptr || out == nullptr) return einval("%s: null pointer", fn);
   if (((reinterpret_cast<uintptr_t>(packed) | reinterpret_cast<uintptr_t>(R) | reinterpret_cast<uintptr_t>(out)) & 15) ||
       (reinterpret_cast<uintptr_t>(scale) & (axis == FADE_AXIS_CHANNEL ? 15 : 1)))
