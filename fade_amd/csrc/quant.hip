@@ -310,15 +310,13 @@ __global__ __launch_bounds__(kBlock) void quant_token_kernel(const InT* __restri
       }
     } else if constexpr (kPkBf) {
       if (on) raw = *reinterpret_cast<const uint4*>(src);
-      fin = finite8_bf16(raw);
-      const uint32_t u[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[2 * i] = __uint_as_float(u[i] << 16);
-        v[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u);
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) a = absmax_nan(a, v[j]);
+      // the lane's largest magnitude as bf16 bits, which order as the values (NaN above inf)
+      auto mag = [](uint32_t u) { return __builtin_bit_cast(u16x2, u & 0x7FFF7FFFu); };
+      const u16x2 t = __builtin_elementwise_max(__builtin_elementwise_max(mag(raw.x), mag(raw.y)),
+                                                __builtin_elementwise_max(mag(raw.z), mag(raw.w)));
+      const uint32_t mm = t[0] > t[1] ? t[0] : t[1];
+      fin = mm < 0x7F80u;
+      a = bf2f(static_cast<uint16_t>(mm));
     } else {
       if (on) load8(src, v);
 #pragma unroll
@@ -343,6 +341,12 @@ __global__ __launch_bounds__(kBlock) void quant_token_kernel(const InT* __restri
         *reinterpret_cast<uint32_t*>(packed + r * row_bytes + c * 4) = codes4_bf16(raw, iv);
         if (c == 0) scale[r] = sc;
         continue;
+      }
+      const uint32_t u[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[2 * i] = __uint_as_float(u[i] << 16);
+        v[2 * i + 1] = __uint_as_float(u[i] & 0xFFFF0000u);
       }
     }
     int code[8];
