@@ -204,37 +204,34 @@ struct Plan {
   int64_t n, tps, n_f16_tiles, tiles_per_split;
 };
 
-// Splits of `tiles` tiles for the packed kernel, `pairs` workgroups per split: at
-// most the count that fills the resident workgroup slots (large caches take
-// it), fewer where the merge costs more than the added workgroups gain.
-// Estimated time in us, from sweeps of forced split counts over B = 1 .. 16 and
-// 600 .. 32K tokens in every format: a wave walks its tiles one at a time, kTile
-// us each (more where two workgroups share a CU, which hides little latency a
-// lone one does not), a further round of workgroups starts over, and a merge
-// costs a round trip through memory plus its splits.  Measured, one-wave rule ->
-// this: B=1, 32/8 heads, 2048 tokens 18.1 -> 9.9 us (34 one-tile splits -> 9),
-// 16K tokens 24.4 -> 16.6 (64 -> 22), B=4 at 4096 15.4 -> 13.2, B=8, 28/4 heads at
-// 470 tokens 11.3 -> 9.7; B=16 at 8192 and the 32K formats as before.
-int64_t packed_splits(int64_t pairs, int64_t tiles, int waves, int resident) {
-  const int64_t cus = num_cus(), per_cu = resident / cus > 0 ? resident / cus : 1;
-  const double kTile = waves == 4 ? 1.55 : 2.0, kShared = 0.5, kStart = 3.0, kMerge = 1.0, kSplit = 0.25;
-  int64_t most = (resident + pairs / 2) / pairs;
-  if (most > tiles) most = tiles;
+// Splits of `tiles` tiles for the packed kernel, `pairs` workgroups per split; `most`
+// splits fill the resident workgroup slots.  Large caches take them all.  Where
+// they leave every wave at most one tile, fewer splits are taken if the merge
+// costs more than the added workgroups gain, as far as a wave still holds one
+// tile: the probabilities are rounded to 16 bits against the maximum of a
+// wave's tiles, so each tile's come out the same in any such plan, and no claim
+// order enters the result.  (With longer splits small calls were faster still, B=1,
+// 32/8 heads, 16K tokens 16.1 us of 23.9, but up to 10% further from a 64-bit softmax,
+// B=2 at 8916 tokens 2.63e-4 -> 2.90e-4, and no longer equal from call to call.)
+// Estimated time in us, from sweeps of forced split counts: a wave's tile takes
+// kTile, longer beside the other waves of its workgroup and a second workgroup of
+// its CU; a merge costs a round trip through memory plus its splits.  Measured,
+// all slots -> this: B=1, 32/8 heads, 657 tokens 10.8 -> 8.7 us, 2048 18.0 -> 9.7
+// (34 one-tile splits -> 9), 4096 16.8 -> 12.3, 8192 19.7 -> 17.5; B=4 at 1030 12.1 -> 9.9; B=8,
+// 28/4 heads at 470 11.2 -> 9.8; rotated 2-bit at 2048 22.1 -> 13.4.
+int64_t packed_splits(int64_t pairs, int64_t tiles, int64_t most, int waves) {
+  if (cdiv(tiles, most) > waves) return most;
+  const double kTile = waves == 4 ? 1.55 : 2.0, kShared = 0.5, kMerge = 1.0, kSplit = 0.25;
   int64_t best = 1;
   double best_us = 0.0;
-  for (int64_t want = 1; want <= most;) {
-    const int64_t per = cdiv(tiles, want), n = cdiv(tiles, per), on_cu = cdiv(pairs * n, cus);
-    const int64_t rounds = on_cu / per_cu, rest = on_cu % per_cu;
-    // tiles of a wave: the waves claim them one at a time, so between the mean and its ceiling
-    const double walk = 0.5 * (static_cast<double>(cdiv(per, waves)) + static_cast<double>(per) / waves);
-    auto round_us = [&](int64_t g) { return kStart + walk * kTile * (1.0 + kShared * (g - 1)); };
-    const double us = rounds * round_us(per_cu) + (rest > 0 ? round_us(rest) : 0.0) + (n > 1 ? kMerge + kSplit * n : 0.0);
-    if (want == 1 || us < best_us) {
+  for (int64_t per = waves; per >= cdiv(tiles, most); --per) {
+    const int64_t n = cdiv(tiles, per), on_cu = cdiv(pairs * n, num_cus());
+    const double walk = 0.5 * (1.0 + static_cast<double>(per) / waves) * kTile;
+    const double us = walk * (1.0 + kShared * (on_cu - 1)) + (n > 1 ? kMerge + kSplit * n : 0.0);
+    if (per == waves || us < best_us) {
       best = n;
       best_us = us;
     }
-    if (per == 1) break;
-    want = cdiv(tiles, per - 1);  // the next count that leaves fewer tiles to a split
   }
   return best;
 }
@@ -246,22 +243,24 @@ Plan make_plan(const fade_decode_args* a, const Params& p) {
     // tiles of either kind cost about the same bytes (8 KB), so splits take equal tile counts
     const int64_t nT = int4_tiles(p);
     const int64_t pairs = a->B * a->Hkv * int4_grid_passes(p);  // workgroups per split
-    int64_t want = a->n_splits > 0 ? a->n_splits : packed_splits(pairs, nT, int4_waves(p), int4_resident_wgs(p));
+    int64_t want = a->n_splits > 0 ? a->n_splits : (int4_resident_wgs(p) + pairs / 2) / pairs;
+    auto plan = [&](int64_t most, int64_t tiles) {  // splits of `tiles`, at most `most`
+      most = most > tiles ? tiles : most;
+      most = most < 1 ? 1 : most;
+      return a->n_splits > 0 || tiles == 0 ? most : packed_splits(pairs, tiles, most, int4_waves(p));
+    };
     pl.n_f16_tiles = int4_fp16_tiles(p);
     pl.tps = 0;
     if (p.rot != nullptr) {
       // rotated middle tier: split 0 = the fp16 tiles, then middle splits of equal tile counts
       const int64_t nMt = nT - pl.n_f16_tiles;
-      int64_t ms = want - 1;
-      if (ms > nMt) ms = nMt;
-      if (ms < 1) ms = 1;
+      int64_t ms = plan(want - 1, nMt);
       if (p.mid.pages != nullptr && ms < cdiv(nMt, kPageSlots)) ms = cdiv(nMt, kPageSlots);
       pl.tiles_per_split = cdiv(nMt, ms);
       pl.n = 1 + cdiv(nMt, pl.tiles_per_split);
       return pl;
     }
-    if (want > nT) want = nT;
-    if (want < 1) want = 1;
+    want = plan(want, nT);
     // paged middle tier: a split's page ids fit the workgroup's kPageSlots
     if (p.mid.pages != nullptr && want < cdiv(nT, kPageSlots)) want = cdiv(nT, kPageSlots);
     pl.tiles_per_split = cdiv(nT, want);
