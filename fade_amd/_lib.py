@@ -272,6 +272,14 @@ def current_stream_handle(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def stream_object(handle: int, device: torch.device) -> torch.cuda.Stream:
+    """The stream of a raw handle.  The default stream's handle is 0, for which
+    ``ExternalStream`` returns a stream of torch's pool instead."""
+    if handle == 0:
+        return torch.cuda.default_stream(device)
+    return torch.cuda.ExternalStream(handle, device=device)
+
+
 def require_gpu(*tensors: torch.Tensor | None, op: str = "fade_amd") -> None:
     """Reject CPU tensors: the hot path has no CPU implementation."""
     dev = None
@@ -350,8 +358,7 @@ def stream_workspace(nbytes: int, device: torch.device, stream: int, pairs: int)
     need = max(int(nbytes), 1)
     ws = _STREAM_WS.get(key)
     if ws is None or ws.numel() < need:
-        target = torch.cuda.ExternalStream(int(stream), device=torch.device("cuda", idx))
-        with torch.cuda.stream(target):
+        with torch.cuda.stream(stream_object(int(stream), torch.device("cuda", idx))):
             if torch.cuda.is_current_stream_capturing():
                 raise RuntimeError(
                     "tiered decode: its shared workspace would be created or grown during HIP-graph capture; "
