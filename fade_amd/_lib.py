@@ -330,6 +330,12 @@ def scratch(nbytes: int, device: torch.device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
 
 
+def scratch_on(nbytes: int, device: torch.device, stream: int) -> torch.Tensor:
+    """``scratch`` for kernels on ``stream``: once dropped, it is used again after them."""
+    with torch.cuda.stream(stream_object(stream, device)):
+        return scratch(nbytes, device)
+
+
 _STREAM_WS: dict = {}  # (device, stream, counter slots) -> the current zero-filled buffer
 _STREAM_WS_OUTGROWN: list = []  # replaced buffers, kept alive for graphs that captured them
 

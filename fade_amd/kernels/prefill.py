@@ -24,8 +24,9 @@ _MASKS = {"bottom_right": _lib.MASK_BOTTOM_RIGHT, "top_left": _lib.MASK_TOP_LEFT
 
 class TieredPrefillPlan:
     """Validated launch for fixed tensors; ``run()`` enqueues one kernel, or two where
-    the keys are split over workgroups (calls too small to fill the GPU; the plan keeps
-    the workspace of their partial sums, so runs of one plan must not overlap).
+    the keys are split over workgroups (calls too small to fill the GPU). The plan keeps
+    the workspace of their partial sums for runs on the stream that it was made on; a
+    run on another stream takes one of its own.
 
     Args:
         q: [B, Hq, Sq, D] fp16 or bf16 queries of the chunk; D a multiple of 8 up to 256.
@@ -131,8 +132,8 @@ class TieredPrefillPlan:
     def run(self, stream: int | None = None) -> Tensor:
         s = torch.cuda.current_stream(self.out.device).cuda_stream if stream is None else stream
         ws = self.workspace
-        if ws is not None and s != self._ws_stream:  # not reused before that stream is done with it
-            ws.record_stream(torch.cuda.ExternalStream(s, device=self.out.device))
+        if ws is not None and s != self._ws_stream:  # not the plan's: overlapping runs, and the plan dropped before this one is done
+            ws = _lib.scratch_on(ws.numel(), self.out.device, s)
         _lib.check(self._fn(self._argp, None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), s),
                    "fade_tiered_prefill_attn")
         return self.out

@@ -113,6 +113,29 @@ def test_prefill_split_on_another_stream(dev):
     assert all(torch.equal(o, want) for o in outs)
 
 
+def test_prefill_split_on_the_default_stream(dev):
+    """A plan made on a side stream, run on the default stream and dropped at once: what is
+    allocated on the side stream next does not overwrite its sums."""
+    plan = _plan(dev, 1, 4, 1, 128, 16, [(4, 1000, 64)], torch.float16, "bottom_right")
+    want, args = plan.run().clone(), plan._keep
+    side, busy = torch.cuda.Stream(), torch.randn(4096, 4096, device=dev)
+    torch.cuda.synchronize()
+    outs = []
+    for _ in range(10):
+        with torch.cuda.stream(side):
+            p = TieredPrefillPlan(*args[:5], lens=args[5])
+        torch.cuda.current_stream().wait_stream(side)
+        busy @ busy  # the run starts after the fill below would
+        outs.append(p.run())
+        n = p.workspace.numel()
+        outs[-1].record_stream(torch.cuda.current_stream())
+        del p
+        with torch.cuda.stream(side):
+            torch.full((n,), 255, dtype=torch.uint8, device=dev)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, want) for o in outs)
+
+
 def test_prefill_split_captured(dev):
     """A captured split call replays to the eager result."""
     plan = _plan(dev, 1, 14, 2, 64, 70, [(4, 2000, 61)], torch.float16, "bottom_right")

@@ -43,3 +43,17 @@ def test_decode_workspace_is_zeroed_on_its_stream(streams):
     _lib.stream_workspace(100, dev, 0, 8)  # the same buffer
     _lib.stream_workspace(100, dev, 0x1234, 8)
     assert streams == [("default", 3), ("external", 0x1234)]
+
+
+def test_prefill_sums_live_on_the_stream_of_the_run(streams):
+    from fade_amd.kernels.prefill import TieredPrefillPlan
+
+    plan = object.__new__(TieredPrefillPlan)
+    plan.out, plan.workspace, plan._ws_stream, plan._argp = torch.full((1,), 0), torch.full((64,), 0, dtype=torch.uint8), 0x55, None
+    calls = []
+    plan._fn = lambda argp, ws, n, stream: calls.append((ws == plan.workspace.data_ptr(), n, stream)) or 0
+    plan.run(0x55)  # the plan's own
+    plan.run(0)
+    plan.run(0x77)
+    assert calls == [(True, 64, 0x55), (False, 64, 0), (False, 64, 0x77)]
+    assert streams == [("default", None), ("external", 0x77)]
