@@ -320,19 +320,20 @@ FADE_API int fade_append_rows(const void* k, int64_t ksb, int64_t ksh, int64_t k
   if (elem_bytes != 2 && elem_bytes != 4) return einval("%s: elements of 2 or 4 bytes, got %lld", fn, (long long)elem_bytes);
   if (at > cap || n > cap - at) return einval("%s: rows %lld..%lld of a buffer of %lld", fn, (long long)at, (long long)(at + n), (long long)cap);
   if (B * H > 65535) return einval("%s: B*H must be at most 65535", fn);
-  if (B * H * n * D == 0) return FADE_OK;
-  if (!k || !v || !buf_k || !buf_v || !buf_pos) return einval("%s: null pointer", fn);
+  if (n == 0) return FADE_OK;
+  const bool rows = B * H * D > 0;  // an empty batch appends its positions only
+  if (!buf_pos || (rows && (!k || !v || !buf_k || !buf_v))) return einval("%s: null pointer", fn);
   const int64_t per = 16 / elem_bytes;  // elements of a unit
   if ((reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(buf_k) |
        reinterpret_cast<uintptr_t>(buf_v)) & 15 ||
       (reinterpret_cast<uintptr_t>(buf_pos) & 7) || (D | ksb | ksh | kss | vsb | vsh | vss) % per)
     return einval("%s: rows must be whole 16-byte units", fn);
-  if (n * (D / per) >= (int64_t{1} << 31)) return einval("%s: too many rows", fn);
+  if (n >= (int64_t{1} << 31) || n * (D / per) >= (int64_t{1} << 31)) return einval("%s: too many rows", fn);
   const AppendArgs a{static_cast<const uint4*>(k), static_cast<const uint4*>(v), ksb / per, ksh / per, kss / per,
                      vsb / per, vsh / per, vss / per, static_cast<uint4*>(buf_k), static_cast<uint4*>(buf_v), buf_pos,
-                     H, cap, at, pos0, static_cast<uint32_t>(n), static_cast<uint32_t>(D / per)};
-  const int64_t blocks = cdiv(n * (D / per), 256);
-  hipLaunchKernelGGL(append_kernel, dim3(static_cast<unsigned>(blocks < 1024 ? blocks : 1024), static_cast<unsigned>(B * H)),
+                     rows ? H : 1, cap, at, pos0, static_cast<uint32_t>(n), rows ? static_cast<uint32_t>(D / per) : 0u};
+  const int64_t blocks = cdiv(rows ? n * (D / per) : n, 256);
+  hipLaunchKernelGGL(append_kernel, dim3(static_cast<unsigned>(blocks < 1024 ? blocks : 1024), static_cast<unsigned>(rows ? B * H : 1)),
                      dim3(256), 0, as_stream(stream), a);
   return check_launch(fn);
 }

@@ -205,7 +205,7 @@ int fade_rerope_gather_dtype(const void* k, int64_t ksb, int64_t ksh, int64_t ks
 /* Append n rows to the full-precision tier's buffers (fade/cache.py:608-670):
  * k, v [B,H,n,D] (element strides, contiguous rows) to rows at .. at + n - 1 of
  * buf_k, buf_v [B,H,cap,D] contiguous, positions pos0 .. pos0 + n - 1 to
- * buf_pos[at ..].  Elements of 2 or 4 bytes; rows are whole 16-byte units
+ * buf_pos[at ..] (also where B, H or D is 0).  Elements of 2 or 4 bytes; rows are whole 16-byte units
  * (pointers 16-byte aligned, D and strides multiples of 16 / elem_bytes). */
 int fade_append_rows(const void* k, int64_t ksb, int64_t ksh, int64_t kss, const void* v, int64_t vsb, int64_t vsh,
                      int64_t vss, int64_t elem_bytes, int64_t B, int64_t H, int64_t n, int64_t D, void* buf_k,

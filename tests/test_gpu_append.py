@@ -66,3 +66,22 @@ def test_append_grows_and_counts_positions(dev):
     full = torch.cat(parts, -2)
     assert torch.equal(ko, full) and torch.equal(vo, -full)
     assert c._layers[0].fp16_pos.tolist() == list(range(330))
+
+
+# no rows of K or V to copy: the positions are appended all the same
+@pytest.mark.parametrize("B,H,D", [(0, 2, 64), (2, 0, 64), (2, 3, 0)])
+def test_append_of_an_empty_batch(dev, B, H, D):
+    k = torch.zeros(B, H, 5, D, device=dev).half()
+    bk, bv, bp = _buffers(B, H, 9, D, torch.float16, dev)
+    if not fc._append_rows(k, k, bk, bv, bp, 2, 70):  # left to the tensor ops
+        return
+    assert bp.tolist() == [-1, -1, 70, 71, 72, 73, 74, -1, -1]
+
+
+def test_update_with_an_empty_batch(dev):
+    c = fc.TieredKVCache(n_sink=2, recent_window=4, head_dim=64)
+    torch.full((1 << 12,), 77, dtype=torch.long, device=dev)  # freed: what an unwritten buffer may hold
+    for n in (300, 1, 1):
+        t = torch.zeros(0, 3, n, 64, device=dev).half()
+        assert c.update(t, t, 0)[0].shape[0] == 0
+    assert c._layers[0].fp16_pos.tolist() == list(range(302))
