@@ -157,6 +157,10 @@ def _append_rows(k: Tensor, v: Tensor, bk: Tensor, bv: Tensor, bp: Tensor, at: i
     kp, vp = k.data_ptr(), v.data_ptr()
     if (kp | vp | bk.data_ptr() | bv.data_ptr()) % 16 or not (bk.is_contiguous() and bv.is_contiguous()):
         return False
+    if not bk.is_inference():  # an in-place write, to autograd as well
+        torch.autograd.graph.increment_version((bk, bv, bp))
+    elif not torch.is_inference_mode_enabled():
+        return False
     _lib.call("fade_append_rows", kp, ks[0], ks[1], ks[2], vp, vs[0], vs[1], vs[2], es, B, H, n, D, bk.data_ptr(),
               bv.data_ptr(), bp.data_ptr(), bk.shape[2], at, pos0, _lib.current_stream_handle(k.device))
     return True

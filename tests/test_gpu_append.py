@@ -85,3 +85,22 @@ def test_update_with_an_empty_batch(dev):
         t = torch.zeros(0, 3, n, 64, device=dev).half()
         assert c.update(t, t, 0)[0].shape[0] == 0
     assert c._layers[0].fp16_pos.tolist() == list(range(302))
+
+
+def test_append_counts_as_an_inplace_write(dev):
+    """What autograd refused of the copies it refuses of the kernel: a backward over tiers that were
+    appended to since, and writes to inference tensors outside inference mode."""
+    r = lambda n: torch.randn(1, 2, n, 64, device=dev).half()  # noqa: E731
+    c = fc.TieredKVCache(n_sink=2, recent_window=4, head_dim=64)
+    c.update(r(5), r(5), 0)
+    w = r(5).requires_grad_()
+    out = (w * c._layers[0].fp16_k).sum()
+    c.update(r(1), r(1), 0)
+    with pytest.raises(RuntimeError, match="inplace operation"):
+        out.backward()
+    with torch.inference_mode():
+        c = fc.TieredKVCache(n_sink=2, recent_window=4, head_dim=64)
+        c.update(r(5), r(5), 0)
+        c.update(r(1), r(1), 0)
+    with pytest.raises(RuntimeError, match="[Ii]nference"):
+        c.update(r(1), r(1), 0)
