@@ -139,9 +139,11 @@ def _sel(x: Tensor, idx: Tensor) -> Tensor:
 def _append_rows(k: Tensor, v: Tensor, bk: Tensor, bv: Tensor, bp: Tensor, at: int, pos0: int) -> bool:
     """Rows ``k``, ``v`` into the buffers from row ``at`` on and their positions, in one
     launch (``fade_append_rows``).  False, with nothing done, for what that kernel does not
-    copy as it is: other devices or dtypes than the buffers', rows that are not whole 16-byte
+    copy as it is: other devices than the current one, other dtypes than the buffers', rows that are not whole 16-byte
     units, tensors that record gradients, subclasses and tracing."""
     if not (k.is_cuda and k.device == v.device == bk.device and _lib.plain(k, v, bk, bv)):
+        return False
+    if k.device.index != torch.cuda.current_device():  # the default stream's handle is the current device's
         return False
     es = k.element_size()
     if k.dtype != bk.dtype or v.dtype != bv.dtype or k.dtype != v.dtype or es not in (2, 4):

@@ -104,3 +104,12 @@ def test_append_counts_as_an_inplace_write(dev):
         c.update(r(1), r(1), 0)
     with pytest.raises(RuntimeError, match="[Ii]nference"):
         c.update(r(1), r(1), 0)
+
+
+def test_append_off_the_current_device(dev, monkeypatch):
+    """Tensors of another device than the current one, on whose streams a launch would go, take the copies."""
+    k = torch.randn(1, 2, 3, 64, device=dev).half()
+    bk, bv, bp = _buffers(1, 2, 8, 64, torch.float16, dev)
+    assert fc._append_rows(k, k, bk, bv, bp, 0, 0)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert not fc._append_rows(k, k, bk, bv, bp, 3, 3)
