@@ -299,8 +299,11 @@ def require_gpu(*tensors: torch.Tensor | None, op: str = "fade_amd") -> None:
 
 def plain(*tensors: torch.Tensor) -> bool:
     """Whether a kernel may stand in for tensor ops on these: plain tensors that record no
-    gradient, outside forward-mode, functorch transforms and compilation."""
+    gradient, outside forward-mode, functorch transforms, compilation, tracing and dispatch
+    modes (which would have seen the ops)."""
     if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    if torch._C._is_tracing() or torch._C._len_torch_dispatch_stack():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
