@@ -298,9 +298,9 @@ def require_gpu(*tensors: torch.Tensor | None, op: str = "fade_amd") -> None:
 
 
 def plain(*tensors: torch.Tensor) -> bool:
-    """Whether a kernel may stand in for tensor ops on these: plain tensors that record no
-    gradient, outside forward-mode, functorch transforms, compilation, tracing and dispatch
-    modes (which would have seen the ops)."""
+    """Whether a kernel may stand in for tensor ops on these: plain tensors whose memory holds
+    their values and that record no gradient, outside forward-mode, functorch transforms,
+    compilation, tracing and dispatch modes (which would have seen the ops)."""
     if torch.compiler.is_compiling() or torch.autograd.forward_ad._current_level >= 0:
         return False
     if torch._C._is_tracing() or torch._C._len_torch_dispatch_stack():
@@ -310,6 +310,8 @@ def plain(*tensors: torch.Tensor) -> bool:
         if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
             return False
         if (grad and t.requires_grad) or torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return False
+        if t.is_neg() or t.is_conj():
             return False
     return True
 

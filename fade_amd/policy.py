@@ -11,6 +11,7 @@ import numpy as np
 import torch
 from torch import Tensor
 
+from ._lib import plain
 from .cache import TIER_EVICT, TIER_FP16, TIER_INT2, TIER_INT4
 
 
@@ -59,12 +60,14 @@ def _assign_one_layer(
 def _top_masks(scores: Tensor, lo: int, hi: int, k1: int, k2: int):
     """Masks over ``scores[lo:hi]`` of its ``k1`` largest values and of the ``k2`` after
     them, by selection instead of a sort (the rule over 4096 host scores: 260 -> 64 us); None where
-    a sort has to decide: device scores, equal values across a boundary, NaN."""
+    a sort has to decide: device scores, equal values across a boundary, NaN, tensors that are
+    no plain memory or are being traced."""
     if scores.device.type != "cpu" or scores.dim() != 1 or int(scores.shape[0]) < hi or k1 < 0:
         return None
-    if scores.dtype not in (torch.float32, torch.float64):
+    scores = scores.detach()
+    if scores.dtype not in (torch.float32, torch.float64) or not plain(scores):
         return None
-    s = scores.detach()[lo:hi].numpy()
+    s = scores[lo:hi].numpy()
     cuts = [c for c in (s.size - k1, s.size - k1 - k2) if c < s.size]
     part = np.partition(s, cuts) if cuts else s
     top = s >= part[s.size - k1] if k1 > 0 else np.zeros(s.size, dtype=bool)

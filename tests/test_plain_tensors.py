@@ -43,3 +43,8 @@ def test_not_plain_while_something_records():
     torch.func.jvp(f("jvp"), (x,), (x,))
     assert seen == dict.fromkeys(seen, False) and len(seen) == 7
     assert _lib.plain(x)
+
+
+def test_not_plain_where_memory_is_not_the_value():
+    assert not _lib.plain(torch.ones(4, dtype=torch.complex64).conj().imag)
+    assert not _lib.plain(torch.ones(4, dtype=torch.complex64).conj())

@@ -51,3 +51,13 @@ def test_assignment_equals_the_sort(S, n_sink, recent, b4, b2):
 def test_scores_shorter_than_the_cache():
     with pytest.raises(IndexError):
         _assign_one_layer(100, torch.rand(50), 4, 4, 10, 0)
+
+
+def test_scores_that_numpy_does_not_take():
+    """Scores with a pending negation, and scores under a recorder: the sort decides, as for other tensors."""
+    z = torch.complex(torch.rand(50), torch.rand(50))
+    s = z.conj().imag
+    assert s.is_neg()
+    assert torch.equal(_assign_one_layer(50, s, 4, 4, 10, 5), _by_sort(50, s, 4, 4, 10, 5))
+    s = torch.rand(50, requires_grad=True)
+    assert torch.equal(_assign_one_layer(50, s, 4, 4, 10, 5), _by_sort(50, s.detach(), 4, 4, 10, 5))
