@@ -128,6 +128,17 @@ __device__ __forceinline__ u32x4 finite_only(u32x4 v) {
   return v;
 }
 
+// The next 16-bit piece of a value of R; a keeps the rest.  A value that is not finite
+// is one piece, and one that rounds to the type's inf starts with its largest.
+template <bool BF>
+__device__ __forceinline__ uint16_t piece(float& a) {
+  uint16_t p = f2w<BF>(a);
+  const bool finite = fabsf(a) < INFINITY;
+  if (finite && (p & 0x7FFFu) == (BF ? 0x7F80u : 0x7C00u)) --p;
+  a = finite ? a - w2f<BF>(p) : 0.0f;
+  return p;
+}
+
 // Work item `it` of a wave: 32 NT rows of one (b, h) slice (per-channel scales),
 // or of the flattened rows (per-token scales: one slice).
 template <int BITS, bool BF, int NT, bool TOKEN>
@@ -155,7 +166,8 @@ __global__ __launch_bounds__(kThreads) void rotdq_kernel(const uint8_t* __restri
     float4 ra[kBlocks], rb[kBlocks];
     const int pair = tid & 15, quad = (tid >> 4) & 3, rest = tid >> 6;
     float mx = 0.0f;
-    auto abs4 = [](const float4& v) { return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))); };
+    auto mag = [](float v) { return fabsf(v) < INFINITY ? fabsf(v) : 0.0f; };
+    auto abs4 = [&](const float4& v) { return fmaxf(fmaxf(mag(v.x), mag(v.y)), fmaxf(mag(v.z), mag(v.w))); };
     // block i: slots 2 pp, 2 pp + 1 (pp = pair + 16 (k & 3)), output channels 4 (quad + 4 (k >> 2)) ..+ 3
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
@@ -172,9 +184,9 @@ __global__ __launch_bounds__(kThreads) void rotdq_kernel(const uint8_t* __restri
       __syncthreads();
 #pragma unroll
       for (int w = 0; w < kWaves; ++w) mx = fmaxf(mx, red[w]);
-      // 2^e with max|R| 2^e in [512, 1024); an orthogonal R's largest entry is at most 1
-      const int e = (mx > 0.0f && mx < INFINITY) ? 9 - ilogbf(mx) : 0;
-      const int ec = e < -60 ? -60 : (e > 60 ? 60 : e);
+      // 2^e with max|R| 2^e in [512, 1024) (the largest finite entry); an orthogonal R's is at most 1
+      const int e = mx > 0.0f ? 9 - ilogbf(mx) : 0;
+      const int ec = e > 120 ? 120 : e;  // both powers are normal floats
       scale_r = ldexpf(1.0f, ec);
       unscale = ldexpf(1.0f, -ec);
     }
@@ -189,10 +201,8 @@ __global__ __launch_bounds__(kThreads) void rotdq_kernel(const uint8_t* __restri
         float a = fa[jj] * scale_r, b = fb[jj] * scale_r;
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
-          const uint16_t pa = f2w<BF>(a), pb = f2w<BF>(b);
-          *reinterpret_cast<uint32_t*>(&rt[q][row][2 * pp]) = pa | (static_cast<uint32_t>(pb) << 16);
-          a -= w2f<BF>(pa);
-          b -= w2f<BF>(pb);
+          const uint32_t pa = piece<BF>(a), pb = piece<BF>(b);
+          *reinterpret_cast<uint32_t*>(&rt[q][row][2 * pp]) = pa | (pb << 16);
         }
       }
     }

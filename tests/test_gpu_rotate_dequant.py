@@ -95,3 +95,31 @@ def test_rotate_dequant_gradient_of_R(dev):
     R = frq._random_orthogonal(128).to(dev).requires_grad_()
     frq.rotated_dequant_v(packed, scale, R, 4, torch.float16).float().sum().backward()
     assert R.grad is not None and bool(R.grad.isfinite().all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("axis", [_lib.AXIS_CHANNEL, _lib.AXIS_TOKEN])
+@pytest.mark.parametrize("what", ["inf", "nan", "large", "largest"])
+def test_rotate_dequant_extreme_R(dev, axis, dtype, what):
+    """Entries of R that are no piece of 16 bits (inf, NaN, a float32 that rounds to a 16-bit inf)
+    or far from 1: inf, NaN and finite values where the 64-bit product's rounding has them."""
+    packed, scale = _inputs((1, 2, 40, 128), 4, axis, dtype, dev)
+    R = frq._random_orthogonal(128).to(dev)
+    if what == "inf":
+        R[5, 9], R[77, 20], R[78, 20], R[3, 127] = float("inf"), float("inf"), -float("inf"), -float("inf")
+    elif what == "nan":
+        R[5, 9] = float("nan")
+    elif what == "large":
+        R = R * 1e25
+    else:
+        R, scale = torch.zeros_like(R), scale * 2.0**-9
+        R[4, 4], R[6, 7] = 3.4e38, -3.4e38
+    out = frq.rotated_dequant_k(packed, scale, R, 4, dtype).double()
+    x = dequant_sym(packed, scale, 4, dtype).double()
+    ref = torch.where(x.unsqueeze(-1) == 0, torch.where(R.isfinite(), 0.0, float("nan")).double(), x.unsqueeze(-1) * R.double()).sum(-2)
+    rounded = ref.to(dtype).double()
+    assert torch.equal(out.isnan(), rounded.isnan())
+    assert torch.equal(out.isposinf(), rounded.isposinf()) and torch.equal(out.isneginf(), rounded.isneginf())
+    fin = rounded.isfinite()
+    tol = (2.0**-10 if dtype == torch.float16 else 2.0**-7) * ref.abs() + 2.0**-18 * R.abs().nan_to_num(0, 0).max().double() * x.abs().sum(-1, keepdim=True)
+    assert bool(((out - ref).abs() <= tol)[fin].all())
