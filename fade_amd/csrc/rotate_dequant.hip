@@ -7,10 +7,15 @@
 // fp32 copy, the fp32 product, the 16-bit copy): 175 us for 33 M elements, of
 // which the fp32 GEMM takes 95.  Here the codes are dequantized in registers
 // into MFMA operands (one rounding to the output type, the reference's) and
-// the product runs on the 16-bit matrix cores with R split so that nothing
-// fp32 holds is lost: fp16 as R_hi + R_lo at a power-of-two scale that puts
-// max|R| in [512, 1024) (~2^-22 of the largest entry), bf16 as three pieces
-// (24 bits); every product accumulates in fp32.
+// the product runs on the 16-bit matrix cores with R in three pieces of its
+// type, which hold the 24 bits of every entry: bf16 as it is, fp16 at a
+// power-of-two scale that puts max|R| in [2^14, 2^15) (entries below 2^-15 of the
+// largest then end at 2^-39 of it).  Every product accumulates in fp32, the small
+// pieces' first, so that their sums are not rounded at the result's size.
+// Against 64 bits, 16 M outputs of each width and axis: as close as the fp32 GEMM or
+// closer (4-bit fp16 9.2 k outputs not the nearest, the GEMM 20 k).  Two pieces in fp16 take
+// 26 us of 31 for 33 M elements, but miss the last bit of 18% of the entries of an
+// orthogonal R, and their 2-bit outputs were further off than the GEMM's.
 //
 // MFMA (32x32x16): C^T[out channel][row] = (R^T)[out][in] x_rot^T[in][row].
 // Lane (n, h) of the B operand holds row n, input channels 64 h + 8 ks ..+ 7
@@ -19,14 +24,15 @@
 // is stored in LDS in that order, and its rows so that lane (n, h) receives
 // the 16 consecutive output channels 32 mt + 16 h ..+ 15 of row n.
 //
-// NT row tiles of 32 per wave share every R fragment read from LDS: at NT = 2
-// (fp16) those reads take half the MFMA time instead of all of it.  One
-// workgroup of 16 waves per CU: R's pieces and the output stage fill its LDS,
+// One workgroup of 16 waves per CU: R's pieces and the output stage fill its LDS,
 // and four waves per SIMD let one's conversions run under another's MFMAs.
-// Measured (4-bit, per call): 16.5 M elements 12 us, 33 M 26.6 us (3.1 TB/s;
-// the two-step path: 168 us), 66 M 55 us (3.0 TB/s).  Up to 33 M elements the
-// split of R in the prologue and the MFMAs bound it, from 66 M the writes (a
-// variant without them: 40 us; without the MFMAs: no faster).
+// Measured (4-bit fp16, per call): 7.7 M elements 12.6 us, 33 M 31 (2.6 TB/s; the two-step
+// path: 168 us), 66 M 56, 131 M 115.  The MFMAs and the reads of R's fragments from LDS,
+// which take as long, bound it with the split of R in the prologue (7 us of a small
+// call); two row tiles per wave, which share each fragment, took the same time
+// (33 M 32.5, 66 M 56, 131 M 115).
+#include <type_traits>
+
 #include "fade_common.h"
 
 namespace fade {
@@ -41,6 +47,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kD = 128;
 constexpr int kWaves = 16;
 constexpr int kThreads = 64 * kWaves;
+constexpr int kRows = 32;     // rows of a wave's work item
+constexpr int kPieces = 3;    // 16-bit pieces of R
 constexpr int kRPitch = 136;  // halves per R^T row in LDS: 16-byte reads of 8 rows hit distinct banks
 constexpr int kStagePitch = 80;  // bytes per staged row of 32 output channels (64 bytes): likewise
 
@@ -128,30 +136,32 @@ __device__ __forceinline__ u32x4 finite_only(u32x4 v) {
   return v;
 }
 
-// The next 16-bit piece of a value of R; a keeps the rest.  A value that is not finite
-// is one piece, and one that rounds to the type's inf starts with its largest.
-template <bool BF>
-__device__ __forceinline__ uint16_t piece(float& a) {
+// The next 16-bit piece of a value of R; a keeps the rest.  ANY: a value that is not
+// finite is one piece, and one that rounds to the type's inf starts with its largest.
+template <bool BF, bool ANY>
+__device__ __forceinline__ uint32_t piece(float& a) {
   uint16_t p = f2w<BF>(a);
-  const bool finite = fabsf(a) < INFINITY;
-  if (finite && (p & 0x7FFFu) == (BF ? 0x7F80u : 0x7C00u)) --p;
-  a = finite ? a - w2f<BF>(p) : 0.0f;
+  if constexpr (ANY) {
+    const bool finite = fabsf(a) < INFINITY;
+    if (finite && (p & 0x7FFFu) == (BF ? 0x7F80u : 0x7C00u)) --p;
+    a = finite ? a - w2f<BF>(p) : 0.0f;
+  } else {
+    a -= w2f<BF>(p);
+  }
   return p;
 }
 
-// Work item `it` of a wave: 32 NT rows of one (b, h) slice (per-channel scales),
+// Work item `it` of a wave: 32 rows of one (b, h) slice (per-channel scales),
 // or of the flattened rows (per-token scales: one slice).
-template <int BITS, bool BF, int NT, bool TOKEN>
+template <int BITS, bool BF, bool TOKEN>
 __global__ __launch_bounds__(kThreads) void rotdq_kernel(const uint8_t* __restrict__ packed,
                                                          const uint16_t* __restrict__ scale, int64_t S,
                                                          uint32_t blocks, uint32_t items, const float* __restrict__ R,
                                                          uint16_t* __restrict__ out) {
-  constexpr int NP = BF ? 3 : 2;  // pieces of R
   constexpr int LB = kLaneBytes<BITS>;
   constexpr int RB = 2 * LB;  // bytes per packed row
-  constexpr int kWaveRows = 32 * NT;
-  __shared__ __attribute__((aligned(16))) uint16_t rt[NP][kD][kRPitch];
-  __shared__ __attribute__((aligned(16))) uint8_t stage[kWaves][kWaveRows * kStagePitch];
+  __shared__ __attribute__((aligned(16))) uint16_t rt[kPieces][kD][kRPitch];
+  __shared__ __attribute__((aligned(16))) uint8_t stage[kWaves][kRows * kStagePitch];
   __shared__ float red[kWaves];
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -165,9 +175,8 @@ __global__ __launch_bounds__(kThreads) void rotdq_kernel(const uint8_t* __restri
     constexpr int kBlocks = kD / 2 * kD / 4 / kThreads;  // 2 x 4 blocks per thread
     float4 ra[kBlocks], rb[kBlocks];
     const int pair = tid & 15, quad = (tid >> 4) & 3, rest = tid >> 6;
-    float mx = 0.0f;
-    auto mag = [](float v) { return fabsf(v) < INFINITY ? fabsf(v) : 0.0f; };
-    auto abs4 = [&](const float4& v) { return fmaxf(fmaxf(mag(v.x), mag(v.y)), fmaxf(mag(v.z), mag(v.w))); };
+    auto bits = [](float v) { return __float_as_uint(v) & 0x7FFFFFFFu; };  // of magnitudes, which order as they do
+    uint32_t top = 0;
     // block i: slots 2 pp, 2 pp + 1 (pp = pair + 16 (k & 3)), output channels 4 (quad + 4 (k >> 2)) ..+ 3
 #pragma unroll
     for (int i = 0; i < kBlocks; ++i) {
@@ -175,84 +184,90 @@ __global__ __launch_bounds__(kThreads) void rotdq_kernel(const uint8_t* __restri
       const float* src = R + (8 * (pp >> 2)) * kD + j0;
       ra[i] = *reinterpret_cast<const float4*>(src + slot_channel<BITS>(e) * kD);
       rb[i] = *reinterpret_cast<const float4*>(src + slot_channel<BITS>(e + 1) * kD);
-      mx = fmaxf(mx, fmaxf(abs4(ra[i]), abs4(rb[i])));
+      for (const float v : {ra[i].x, ra[i].y, ra[i].z, ra[i].w, rb[i].x, rb[i].y, rb[i].z, rb[i].w}) top = max(top, bits(v));
     }
+    // entries that are inf, NaN or round to a bf16 inf: rare, and split with more care
+    const bool extreme = __builtin_amdgcn_ballot_w64(top >= (BF ? 0x7F7F8000u : 0x7F800000u)) != 0;
     float scale_r = 1.0f;
     if constexpr (!BF) {
+      float mx = __uint_as_float(top);
+      if (extreme) {  // the largest finite entry
+        mx = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kBlocks; ++i)
+          for (const float v : {ra[i].x, ra[i].y, ra[i].z, ra[i].w, rb[i].x, rb[i].y, rb[i].z, rb[i].w})
+            mx = bits(v) < 0x7F800000u ? fmaxf(mx, fabsf(v)) : mx;
+      }
       mx = group_max<64>(mx);
       if (lane == 0) red[wave] = mx;
       __syncthreads();
 #pragma unroll
       for (int w = 0; w < kWaves; ++w) mx = fmaxf(mx, red[w]);
-      // 2^e with max|R| 2^e in [512, 1024) (the largest finite entry); an orthogonal R's is at most 1
-      const int e = mx > 0.0f ? 9 - ilogbf(mx) : 0;
+      // 2^e with max|R| 2^e in [2^14, 2^15) (the largest finite entry); an orthogonal R's is at most 1
+      const int e = mx > 0.0f ? 14 - ilogbf(mx) : 0;
       const int ec = e > 120 ? 120 : e;  // both powers are normal floats
       scale_r = ldexpf(1.0f, ec);
       unscale = ldexpf(1.0f, -ec);
     }
+    auto split = [&](auto any) {
 #pragma unroll
-    for (int i = 0; i < kBlocks; ++i) {
-      const int k = rest + i * kWaves, pp = pair + 16 * (k & 3), j0 = 4 * (quad + 4 * (k >> 2));
-      const float fa[4] = {ra[i].x, ra[i].y, ra[i].z, ra[i].w}, fb[4] = {rb[i].x, rb[i].y, rb[i].z, rb[i].w};
+      for (int i = 0; i < kBlocks; ++i) {
+        const int k = rest + i * kWaves, pp = pair + 16 * (k & 3), j0 = 4 * (quad + 4 * (k >> 2));
+        const float fa[4] = {ra[i].x, ra[i].y, ra[i].z, ra[i].w}, fb[4] = {rb[i].x, rb[i].y, rb[i].z, rb[i].w};
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        // output channel 32 mt + 16 h' + 4 a + b sits in A row 32 mt + 8 a + 4 h' + b
-        const int j = j0 + jj, row = (j & ~31) | (((j >> 2) & 3) << 3) | (((j >> 4) & 1) << 2) | (j & 3);
-        float a = fa[jj] * scale_r, b = fb[jj] * scale_r;
+        for (int jj = 0; jj < 4; ++jj) {
+          // output channel 32 mt + 16 h' + 4 a + b sits in A row 32 mt + 8 a + 4 h' + b
+          const int j = j0 + jj, row = (j & ~31) | (((j >> 2) & 3) << 3) | (((j >> 4) & 1) << 2) | (j & 3);
+          float a = fa[jj] * scale_r, b = fb[jj] * scale_r;
 #pragma unroll
-        for (int q = 0; q < NP; ++q) {
-          const uint32_t pa = piece<BF>(a), pb = piece<BF>(b);
-          *reinterpret_cast<uint32_t*>(&rt[q][row][2 * pp]) = pa | (pb << 16);
+          for (int q = 0; q < kPieces; ++q) {
+            const uint32_t pa = piece<BF, decltype(any)::value>(a), pb = piece<BF, decltype(any)::value>(b);
+            *reinterpret_cast<uint32_t*>(&rt[q][row][2 * pp]) = pa | (pb << 16);
+          }
         }
       }
-    }
+    };
+    if (__builtin_expect(extreme, 0)) split(std::true_type{});
+    else split(std::false_type{});
   }
   __syncthreads();
 
   auto rows_of = [&](uint32_t it, int64_t& slice, int64_t& r0) {  // the wave's first row of item it
     const uint32_t sl = TOKEN ? 0u : it / blocks;
     slice = sl;
-    r0 = static_cast<int64_t>(it - sl * blocks) * kWaveRows;
+    r0 = static_cast<int64_t>(it - sl * blocks) * kRows;
   };
-  auto load = [&](uint32_t it, Codes<BITS> (&cd)[NT], uint32_t (&ts)[NT]) {
+  auto load = [&](uint32_t it, Codes<BITS>& cd, uint32_t& ts) {
     int64_t slice, r0;
     rows_of(it, slice, r0);
+    const int64_t row = slice * S + (r0 + n < S ? r0 + n : S - 1);  // rows past the slice: its last row, never stored
+    const u32x4* src = reinterpret_cast<const u32x4*>(packed + row * RB + h * LB);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int64_t rr = r0 + 32 * t + n;
-      const int64_t row = slice * S + (rr < S ? rr : S - 1);  // rows past the slice: its last row, never stored
-      const u32x4* src = reinterpret_cast<const u32x4*>(packed + row * RB + h * LB);
-#pragma unroll
-      for (int k = 0; k < LB / 16; ++k) cd[t].w[k] = src[k];
-      ts[t] = TOKEN ? scale[row] : 0u;
-    }
+    for (int k = 0; k < LB / 16; ++k) cd.w[k] = src[k];
+    ts = TOKEN ? scale[row] : 0u;
   };
 
   // neighbouring items go to different workgroups, so a few of them spread over the CUs
   for (uint32_t it = wave * gridDim.x + blockIdx.x; it < items; it += kWaves * gridDim.x) {
-    Codes<BITS> cd[NT];
-    uint32_t ts[NT];
+    Codes<BITS> cd;
+    uint32_t ts;
     load(it, cd, ts);
     __asm__ volatile("" ::: "memory");  // keep the R fragment reads inside the loop
     int64_t slice, r0;
     rows_of(it, slice, r0);
-    u32x4 x[NT][8];
+    u32x4 x[8];
     bool big = false;
     if constexpr (TOKEN) {
+      const uint32_t s2 = ts | (ts << 16);
+      big = big_scale<BF>(ts);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const uint32_t s2 = ts[t] | (ts[t] << 16);
-        big |= big_scale<BF>(ts[t]);
+      for (int ks = 0; ks < 8; ++ks) {
+        f16x2 c[4];
+        codes8<BITS>(cd, ks, c);
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-          f16x2 c[4];
-          codes8<BITS>(cd[t], ks, c);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) x[t][ks][j] = scaled<BF>(c[j], s2);
-        }
+        for (int j = 0; j < 4; ++j) x[ks][j] = scaled<BF>(c[j], s2);
       }
-    }
-    else {
+    } else {
       const u32x4* sp = reinterpret_cast<const u32x4*>(scale + slice * kD + 64 * h);
 #pragma unroll
       for (int ks = 0; ks < 8; ++ks) {
@@ -263,14 +278,11 @@ __global__ __launch_bounds__(kThreads) void rotdq_kernel(const uint8_t* __restri
           sv[j] = (sw[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
           big |= big_scale<BF>(sv[j]);
         }
+        f16x2 c[4];
+        codes8<BITS>(cd, ks, c);
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          f16x2 c[4];
-          codes8<BITS>(cd[t], ks, c);
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            x[t][ks][j] = scaled<BF>(c[j], sv[slot_channel<BITS>(2 * j)] | (sv[slot_channel<BITS>(2 * j + 1)] << 16));
-        }
+        for (int j = 0; j < 4; ++j)
+          x[ks][j] = scaled<BF>(c[j], sv[slot_channel<BITS>(2 * j)] | (sv[slot_channel<BITS>(2 * j + 1)] << 16));
       }
     }
     // inf times a piece of R of either sign would give NaN where the whole
@@ -279,53 +291,43 @@ __global__ __launch_bounds__(kThreads) void rotdq_kernel(const uint8_t* __restri
     const bool any_big = __builtin_amdgcn_ballot_w64(big) != 0;
 #pragma unroll 1
     for (int mt = 0; mt < 4; ++mt) {
-      f32x16 acc[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] = f32x16{};
+      // the small pieces' sums first: rounded at their own size, not at the result's
+      f32x16 acc = {};
       if (__builtin_expect(!any_big, 1)) {
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
+        for (int q = kPieces - 1; q >= 0; --q)
 #pragma unroll
-          for (int q = 0; q < NP; ++q) {
-            const u32x4 a = *reinterpret_cast<const u32x4*>(&rt[q][32 * mt + n][64 * h + 8 * ks]);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) acc[t] = mfma<BF>(a, x[t][ks], acc[t]);
-          }
+          for (int ks = 0; ks < 8; ++ks)
+            acc = mfma<BF>(*reinterpret_cast<const u32x4*>(&rt[q][32 * mt + n][64 * h + 8 * ks]), x[ks], acc);
       } else {
 #pragma unroll 1
-        for (int q = 0; q < NP; ++q) {
+        for (int q = kPieces - 1; q >= 0; --q) {
 #pragma unroll
           for (int ks = 0; ks < 8; ++ks) {
-            const u32x4 a = *reinterpret_cast<const u32x4*>(&rt[q][32 * mt + n][64 * h + 8 * ks]);
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-              u32x4 xv = x[t][ks];
-              __asm__ volatile("" : "+v"(xv));  // computed here, in this rare branch, not ahead of the loop
-              acc[t] = mfma<BF>(a, q == 0 ? xv : finite_only<BF>(xv), acc[t]);
-            }
+            u32x4 xv = x[ks];
+            __asm__ volatile("" : "+v"(xv));  // computed here, in this rare branch, not ahead of the loop
+            acc = mfma<BF>(*reinterpret_cast<const u32x4*>(&rt[q][32 * mt + n][64 * h + 8 * ks]),
+                           q == 0 ? xv : finite_only<BF>(xv), acc);
           }
         }
       }
-      // lane (n, h): channels 32 mt + 16 h ..+ 15 of row n of each tile -> the wave's stage
+      // lane (n, h): channels 32 mt + 16 h ..+ 15 of row n -> the wave's stage
       uint8_t* const st = &stage[wave][0];
+      u32x4 o[2];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        u32x4 o[2];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float a = acc[t][2 * j] * unscale, b = acc[t][2 * j + 1] * unscale;
-          o[j >> 2][j & 3] = BF ? pack_bf16(a, b) : static_cast<uint32_t>(f2h(a)) | (static_cast<uint32_t>(f2h(b)) << 16);
-        }
-        u32x4* dst = reinterpret_cast<u32x4*>(st + (32 * t + n) * kStagePitch + 32 * h);
-        dst[0] = o[0];
-        dst[1] = o[1];
+      for (int j = 0; j < 8; ++j) {
+        const float a = acc[2 * j] * unscale, b = acc[2 * j + 1] * unscale;
+        o[j >> 2][j & 3] = BF ? pack_bf16(a, b) : static_cast<uint32_t>(f2h(a)) | (static_cast<uint32_t>(f2h(b)) << 16);
       }
+      u32x4* dst = reinterpret_cast<u32x4*>(st + n * kStagePitch + 32 * h);
+      dst[0] = o[0];
+      dst[1] = o[1];
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       // out in whole 64-byte row segments
 #pragma unroll
-      for (int k = 0; k < 2 * NT; ++k) {
+      for (int k = 0; k < 2; ++k) {
         const int rr = 16 * k + (lane >> 2);
         const u32x4 v = *reinterpret_cast<const u32x4*>(st + rr * kStagePitch + 16 * (lane & 3));
         if (r0 + rr < S)
@@ -343,18 +345,9 @@ void launch(const uint8_t* packed, const uint16_t* scale, int64_t BH, int64_t S,
             hipStream_t st) {
   const int64_t slices = TOKEN ? 1 : BH, rows = TOKEN ? BH * S : S;
   const int cus = num_cus();
-  // two row tiles per wave once that still gives every wave of the grid one
-  // (fp16 only: bf16's third piece of R leaves no LDS for the stage, raw int8
-  // 3-bit codes no registers)
-  constexpr int NT = BITS != 3 && !BF ? 2 : 1;
-  const int64_t waves = static_cast<int64_t>(cus) * kWaves;
-  const int nt = slices * cdiv(rows, 32 * NT) >= waves ? NT : 1;
-  const uint32_t blocks = static_cast<uint32_t>(cdiv(rows, 32 * nt)), items = static_cast<uint32_t>(slices * blocks);
+  const uint32_t blocks = static_cast<uint32_t>(cdiv(rows, kRows)), items = static_cast<uint32_t>(slices * blocks);
   const dim3 grid(items < static_cast<uint32_t>(cus) ? items : cus);
-  if (NT == 2 && nt == 2)
-    hipLaunchKernelGGL((rotdq_kernel<BITS, BF, NT, TOKEN>), grid, dim3(kThreads), 0, st, packed, scale, rows, blocks, items, R, out);
-  else
-    hipLaunchKernelGGL((rotdq_kernel<BITS, BF, 1, TOKEN>), grid, dim3(kThreads), 0, st, packed, scale, rows, blocks, items, R, out);
+  hipLaunchKernelGGL((rotdq_kernel<BITS, BF, TOKEN>), grid, dim3(kThreads), 0, st, packed, scale, rows, blocks, items, R, out);
 }
 
 }  // namespace

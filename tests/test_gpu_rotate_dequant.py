@@ -26,8 +26,8 @@ def _inputs(shape, bits, axis, dtype, dev, seed=3):
 
 
 def _check(packed, scale, R, bits, dtype):
-    """|out - exact| <= half an ulp of the output plus the fp32-GEMM term: 128 products, each
-    entry of R carried to 2^-21 of max|R| (2^-24 relative in bf16's three pieces)."""
+    """|out - exact| <= half an ulp of the output plus the fp32-GEMM term: 128 products summed
+    in fp32, each entry of R in its 24 bits."""
     assert frq._dequant_fused_ok(packed, R, bits, dtype)
     out = frq.rotated_dequant_k(packed, scale, R, bits, dtype).double()
     x = dequant_sym(packed, scale, bits, dtype).double()
@@ -38,7 +38,7 @@ def _check(packed, scale, R, bits, dtype):
 
 
 # 33, 70: a second, partly filled 32-row tile; 257, 300: a second item of a workgroup's 256
-# rows; (2, 8, 8200): two row tiles per wave, 8200 % 512 rows left in the last item
+# rows; (2, 8, 8200): more items than the grid's 4096 waves, 8200 % 32 rows left in the last item
 @pytest.mark.parametrize("shape", [(1, 1, 1, 128), (2, 3, 33, 128), (1, 2, 70, 128), (1, 3, 257, 128), (2, 8, 8200, 128)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bits", [4, 3, 2])
@@ -50,6 +50,27 @@ def test_rotate_dequant(dev, bits, dtype, shape):
         _check(packed, scale, R, bits, dtype)
         _check(packed, scale, R * 300.0, bits, dtype)  # entries far above and below an orthogonal matrix's
         _check(packed, scale * 64.0, R * 1e-4, bits, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [4, 3, 2])
+@pytest.mark.parametrize("size", [2.0**-4, 1.0, 2.0**20])  # 2^-4: a scale of 2^14, the careful branch in fp16
+def test_rotate_dequant_last_bits_of_R(dev, bits, dtype, size):
+    """The difference of two rows of R that agree in 21 bits is exact in float32: all 24 bits count."""
+    g = torch.Generator().manual_seed(8)
+    w = torch.rand(128, generator=g) + 1.0
+    R = torch.zeros(128, 128)
+    R[17], R[90] = w, (w.view(torch.int32) & ~7).view(torch.float32)
+    R[3] = torch.rand(128, generator=g)
+    R = (R * size).to(dev)
+    codes = torch.zeros(1, 1, 70, 128, dtype=torch.int8, device=dev)
+    codes[..., 17], codes[..., 90] = 1, -1
+    packed = codes if bits == 3 else frq._pack_codes(codes, bits)
+    scale = torch.full((1, 1, 70, 1), 2.0**10 / size, dtype=dtype, device=dev)
+    out = frq.rotated_dequant_v(packed, scale, R, bits, dtype)
+    want = ((R[17].double() - R[90].double()) * scale.double().flatten()[0]).to(dtype)
+    assert int((want != 0).sum()) > 64
+    assert torch.equal(out, want.expand_as(out))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
