@@ -1391,6 +1391,7 @@ FADE_API int fade_quant_k_int4_polls(const void* k, int32_t dtype, int64_t B, in
                                      int64_t sb, int64_t sh, int64_t ss, int32_t polls, void* packed_u8, void* scale,
                                      void* workspace, int64_t workspace_bytes, void* stream) {
   const char* fn = "fade_quant_k_int4_dtype";
+  if (polls < 0) return einval("%s: polls must not be negative, got %d", fn, polls);
   int rc = check_dims(fn, B, H, S, D);
   if (rc) return rc;
   if (!aligned(k, 16) || (sb | sh | ss) % 8 != 0)

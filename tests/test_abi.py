@@ -174,3 +174,10 @@ def test_argument_errors_come_back_as_value_errors():
     assert b"not a multiple" in lib.fade_hip_last_error()
     rc = lib.fade_quant_int2_grouped(None, 1, 1, 100, 100, 128, 0, 0, 0, 64, None, None, None)
     assert rc == _lib.FADE_EINVAL and b"must be divisible by group_size" in lib.fade_hip_last_error()
+
+
+@pytest.mark.parametrize("polls,rc", [(-1, 1), (-(2**31), 1), (0, 0), (2**31 - 1, 0)])
+def test_poll_bound_is_checked(polls, rc):
+    lib = _lib.load()
+    got = lib.fade_quant_k_int4_polls(None, 0, 0, 8, 64, 128, 64, 64, 128, polls, None, None, None, 0, None)  # an empty batch
+    assert got == (_lib.FADE_EINVAL if rc else _lib.FADE_OK)
