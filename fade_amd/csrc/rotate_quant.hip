@@ -35,10 +35,10 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kD = 128;
 constexpr int kWaves = 8;
 constexpr int kThreads = 64 * kWaves;
-// Waves of the per-token kernel: four per SIMD, no tile loaded ahead (config 2's
-// 1.04 M rows: 81 us; two per SIMD with the next tile in flight 87).  The
-// per-channel passes keep 8 waves with two tiles each per R fragment (163 us for
-// both; 16 waves of one tile: 173).
+// Waves of the per-token kernel: four per SIMD, no tile loaded ahead (1.04 M rows
+// of 2-bit V 74-82 us; two per SIMD with the next tile in flight 86-93, in turn on
+// the same card).  The per-channel passes keep 8 waves with two tiles each per R
+// fragment (150-166 us for both; 16 waves of one tile: 173).
 constexpr int kTokenWaves = 16;
 constexpr int kTokenThreads = 64 * kTokenWaves;
 constexpr int kRows = 32;     // rows per wave tile
@@ -232,9 +232,11 @@ __device__ __forceinline__ void flush_stage(const uint8_t* stage, uint8_t* __res
 
 // Per-token scales: the waves of the grid take 32-row tiles of the flattened
 // [B*H*S] rows in turn.  Bound by the matrix cores and the issue around them:
-// without the loads of x it takes 70 us, with half the MFMAs 69.
+// without the loads of x it takes 70 us, with half the MFMAs 69.  First tile of a
+// wave: block_tile * workgroup + wave_tile * wave.
 template <int BITS>
 __global__ __launch_bounds__(kTokenThreads) void rotq_token_kernel(const uint16_t* __restrict__ x, Geom gm, int64_t rows,
+                                                              int block_tile, int wave_tile,
                                                               const float* __restrict__ R,
                                                               uint8_t* __restrict__ packed,
                                                               uint16_t* __restrict__ scale) {
@@ -245,7 +247,7 @@ __global__ __launch_bounds__(kTokenThreads) void rotq_token_kernel(const uint16_
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 31, h = lane >> 5;
   const int64_t step = static_cast<int64_t>(gridDim.x) * kTokenWaves * kRows;
-  int64_t r0 = (static_cast<int64_t>(blockIdx.x) * kTokenWaves + wave) * kRows;
+  int64_t r0 = static_cast<int64_t>(blockIdx.x * block_tile + wave * wave_tile) * kRows;
   const int64_t last = rows - 1;
   for (; r0 < rows; r0 += step) {
     __asm__ volatile("" ::: "memory");  // keep the R fragment reads inside the loop
@@ -448,14 +450,21 @@ FADE_API int fade_rotate_quant(const void* x_f16, int64_t B, int64_t H, int64_t 
   uint16_t* sc = static_cast<uint16_t*>(scale_f16);
   hipStream_t st = as_stream(stream);
   if (axis == FADE_AXIS_TOKEN) {
-    const int64_t want = cdiv(rows, static_cast<int64_t>(kRows) * kTokenWaves);
-    const int64_t cap = num_cus();
-    const dim3 grid(static_cast<unsigned>(want < cap ? want : cap));
+    const int64_t tiles = cdiv(rows, kRows), cus = num_cus();
+    // up to one tile per wave: neighbouring tiles go to different workgroups, so that a few of
+    // them spread over the CUs (3200 rows 8.9 -> 5.8 us, 32,000 9.4 -> 6.7); with more, a
+    // workgroup's waves read next to each other (1.04 M rows 74 us, spread 80)
+    const bool spread = tiles <= cus * kTokenWaves;
+    const int grid = static_cast<int>(tiles < cus ? tiles : cus);
+    const int bt = spread ? 1 : kTokenWaves, wt = spread ? grid : 1;
+#define FADE_ROTQ_TOKEN(BITS) \
+  hipLaunchKernelGGL(rotq_token_kernel<BITS>, dim3(grid), dim3(kTokenThreads), 0, st, x, gm, rows, bt, wt, R, pk, sc)
     switch (bits) {
-      case 4: hipLaunchKernelGGL(rotq_token_kernel<4>, grid, dim3(kTokenThreads), 0, st, x, gm, rows, R, pk, sc); break;
-      case 3: hipLaunchKernelGGL(rotq_token_kernel<3>, grid, dim3(kTokenThreads), 0, st, x, gm, rows, R, pk, sc); break;
-      default: hipLaunchKernelGGL(rotq_token_kernel<2>, grid, dim3(kTokenThreads), 0, st, x, gm, rows, R, pk, sc); break;
+      case 4: FADE_ROTQ_TOKEN(4); break;
+      case 3: FADE_ROTQ_TOKEN(3); break;
+      default: FADE_ROTQ_TOKEN(2); break;
     }
+#undef FADE_ROTQ_TOKEN
     return check_launch(fn);
   }
   int64_t nsb, rpb;

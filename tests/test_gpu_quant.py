@@ -435,3 +435,16 @@ def test_empty_and_error_inputs(dev):
         fq.quant_v_int4(torch.zeros(1, 1, 4, 100, dtype=torch.float16, device=dev))
     with pytest.raises(ValueError, match="head_dim must be"):
         fq.quant_v_int4(torch.zeros(1, 1, 4, 264, dtype=torch.float16, device=dev))
+
+
+# rows on either side of a tile, of a tile per workgroup and of a tile per wave of the grid
+@pytest.mark.parametrize("bits", [4, 3, 2])
+def test_rotated_quant_v_row_counts(dev, bits):
+    """A row's codes and scale do not depend on how many rows the call has."""
+    g = torch.Generator(device=dev).manual_seed(bits)
+    x = torch.randn(1, 1, 140000, 128, device=dev, generator=g).half()
+    R = frq._random_orthogonal(128).to(dev)
+    packed, scale = frq.rotated_quant_v(x, R, bits)
+    for n in (1, 31, 33, 8192, 8193, 131072, 131073):
+        p, s = frq.rotated_quant_v(x[:, :, :n], R, bits)
+        assert torch.equal(p, packed[:, :, :n]) and torch.equal(s, scale[:, :, :n]), n
