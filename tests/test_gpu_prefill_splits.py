@@ -89,6 +89,35 @@ def test_prefill_key_splits(dev, B, Hq, Hkv, D, Sq, rows, dtype, mask):
     assert torch.equal(plan.run().double(), out)  # merged in a fixed order
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("what", ["K nan", "K inf", "K -inf scores", "V nan", "V inf", "V both infs"])
+def test_prefill_split_non_finite(dev, dtype, what):
+    """inf and NaN in one split's keys reach the merged rows as they reach the unsplit kernel's."""
+    plan = _plan(dev, 2, 4, 2, 128, 40, [(4, 1500, 64), (4, 700, 64)], dtype, "bottom_right")
+    assert plan.workspace is not None
+    q, chunk, sink, mid, rec = plan._keep[:5]
+    inf = float("inf")
+    if what == "K nan":
+        rec[0][0, 1, 7, 5] = float("nan")
+    elif what == "K inf":
+        rec[0][0, 1, 7, 5] = inf
+    elif what == "K -inf scores":  # a key that no query of the group sees
+        q[0, 2:, :, 5] = q[0, 2:, :, 5].abs() + 1
+        rec[0][0, 1, 7, 5] = -inf
+    elif what == "V nan":
+        sink[1][0, 1, 2, 9] = float("nan")
+    elif what == "V inf":
+        sink[1][0, 1, 2, 9] = -inf
+    else:  # +inf and -inf in different splits
+        sink[1][0, 1, 2, 9], rec[1][0, 1, 7, 9] = inf, -inf
+    out, one = plan.run().float(), _unsplit(plan).float()
+    assert torch.equal(out.isnan(), one.isnan()) and torch.equal(out.isposinf(), one.isposinf()) and torch.equal(out.isneginf(), one.isneginf())
+    assert bool(out[1].isfinite().all() and out[0, :2].isfinite().all())
+    assert bool(out.isfinite().all()) == (what == "K -inf scores")
+    fin = out.isfinite()
+    assert bool(((out - one).abs() <= (2e-3 if dtype == torch.float16 else 8e-3) + 2.0**-7 * one.abs())[fin].all())
+
+
 def test_prefill_split_workspace_checked(dev):
     plan = _plan(dev, 1, 4, 1, 128, 16, [(4, 1000, 64)], torch.float16, "bottom_right")
     lib, s = _lib.load(), torch.cuda.current_stream().cuda_stream
