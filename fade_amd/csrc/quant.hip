@@ -1171,7 +1171,11 @@ void channel_blocking(int64_t BH, int64_t S, int64_t* nsb, int64_t* rows_per_blo
 }
 
 // Polls of quant_channel_once_kernel's wait, about 1 us each: far beyond the wait of
-// a slice whose workgroups run together (a few us).
+// a slice whose workgroups run together (a few us).  The way out costs much more than
+// the wait (every workgroup reads its slice: 16 x 8 x 8124 fp16 69 us, 979 if all take it), so
+// the bound also covers workgroups that wait for CUs held by another stream's
+// kernels.  A call beside a stream of them, two passes -> this: chunk prefill 480 ->
+// 422 us (8 polls: 1151), 8192^3 matrix products 728 -> 710, copies 233 -> 132.
 constexpr int kPolls = 256;
 // Inputs of at least half the 256 MB device cache are read with non-temporal loads
 // (266 MB: 71.7 -> 67.9 us; 61 MB, which the cache may hold: 23.0 -> 24.4).
@@ -1182,7 +1186,9 @@ constexpr int64_t kMostWaiting = 128;
 
 // Rows per thread of the single-pass form and its workgroups per (b, h): 64
 // registers of row data, or 16 where that many per thread would leave CUs idle;
-// n = 0: the two-pass form.
+// n = 0: the two-pass form, for slices of more than kMostWaiting workgroups (few long
+// slices among them, 2-byte types from 8193 rows at D = 128, where the form of 64 would
+// have fewer: not tried).
 struct OncePlan {
   bool big;
   int64_t n, words;  // workgroups of a (b, h); dwords of all exchange areas
